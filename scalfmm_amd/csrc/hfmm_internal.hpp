@@ -90,6 +90,12 @@ struct Context {
     DevBuf d_posoff;         // [343] int64 offset of a position's mixed operators in d_opm
     DevBuf d_opm;            // mixed precision: position-specific operators, bf16 hi/mid/lo planes
     DevBuf d_opm2;           // the same with U's rank columns interleaved (wave-level kernel, p <= 6)
+    // FP64 M2L (m2l_f64.hip): rows of all offsets, tables, operator fragments of
+    // the two products, the compressed expansions between them, and the partial
+    // locals of a launch over parts of the rows
+    DevBuf d_m2lrows, d_m2ltab, d_m2lup, d_m2ldown, d_m2lC, d_m2lacc;
+    int m2l_nrb = 0;             // row blocks of 16
+    std::vector<int> m2l_rboff;  // doubles of a target's C before each row block
     int m2l_variant = -1;    // M2L kernel variant; -1: pick by timing at the next M2L
     float m2l_tune_ms[4] = {0.f, 0.f, 0.f, 0.f};  // times measured by the last autotune
 
@@ -277,7 +283,8 @@ int build_p2p_mutual_tables(Context* c);
 // FP64 passes (fmm_device.hip)
 int run_p2m(Context* c);
 int run_m2m(Context* c, int level);  // parents at `level`, children at level+1
-int run_m2l(Context* c);  // every level 2..h-1 in one launch
+int prepare_m2l_f64(Context* c);  // tables and operator fragments of the uploaded operators (m2l_f64.hip)
+int run_m2l(Context* c);          // every level 2..h-1
 int run_l2l(Context* c, int level);  // parents at `level`
 int run_l2p(Context* c);
 int run_p2p(Context* c);

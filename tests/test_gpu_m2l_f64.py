@@ -1,0 +1,43 @@
+"""The FP64 M2L at the edges of its tiles against the oracle: fewer cells than a
+column tile, partly filled tiles, both tile shapes (below and above 16,384
+cells), every order, and sparse trees whose tiles skip offsets.  Locals and
+results to 1e-12 relative L2, the bound of the FP64 path."""
+import numpy as np
+import pytest
+
+from oracle import pyoracle
+from scalfmm_amd import Engine
+from scalfmm_amd.distributions import plummer, uniform_cube
+
+pytestmark = pytest.mark.gpu
+CENTER = (0.5, 0.5, 0.5)
+
+CASES = [
+    (uniform_cube, 9, 3, 5),  # a handful of cells
+    (uniform_cube, 700, 4, 6),  # 585 cells at most: one partly filled tile of the last workgroup
+    (uniform_cube, 701, 4, 7),
+    (uniform_cube, 3001, 4, 8),
+    (plummer, 20011, 6, 5),  # sparse: tiles without some of the offsets
+    (plummer, 20011, 7, 7),
+    (uniform_cube, 45001, 6, 5),  # above 16,384 cells: two column tiles per workgroup
+    (uniform_cube, 45001, 6, 6),
+    (uniform_cube, 45001, 6, 7),
+    (uniform_cube, 45001, 6, 8),
+]
+
+
+def rel(a, b):
+    return np.linalg.norm(a - b) / np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("dist,n,h,p", CASES)
+def test_m2l_tiles(dist, n, h, p):
+    x, y, z, q = dist(n, 17)
+    e = Engine(h, 1.0, CENTER, p)
+    e.set_particles(x, y, z, q)
+    e.build_tree()
+    e.evaluate()
+    ref = pyoracle.fmm(x, y, z, q, CENTER, 1.0, h, p)
+    for got, want in zip(e.results(), ref[:4]):
+        assert rel(got, want) < 1e-12
+    e.close()
