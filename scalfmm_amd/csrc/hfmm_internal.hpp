@@ -95,7 +95,7 @@ struct Context {
     // locals of a launch over parts of the rows
     DevBuf d_m2lrows, d_m2ltab, d_m2lup, d_m2ldown, d_m2lC, d_m2lacc;
     int m2l_nrb = 0;             // row blocks of 16
-    std::vector<int> m2l_rboff;  // doubles of a target's C before each row block
+    std::vector<int> m2l_rboff;  // bytes of a target's C before each row block
     int m2l_variant = -1;    // M2L kernel variant; -1: pick by timing at the next M2L
     float m2l_tune_ms[4] = {0.f, 0.f, 0.f, 0.f};  // times measured by the last autotune
 

@@ -48,8 +48,7 @@ constexpr int kTauStride = 60; // bytes per cell of a table over the offsets (wh
 constexpr int kMWaves = 8;
 constexpr int kMThreads = 64 * kMWaves;
 constexpr int kMaxSteps = 256;  // row blocks: 56 offsets of rank <= 64
-constexpr int kNoSlot = kFarSlots;  // also the entry past a cell's slots in the table of its targets, which holds none
-constexpr int kTgtRow = kFarSlots + 2;
+constexpr int kTgtRow = 8 * (kTau + 1) + 4;  // entries of a source in the table of its targets (rows on other banks)
 constexpr int kXcdChunk = 16;   // consecutive tiles that run on one XCD
 
 // Keeps the scheduler from moving the work of a phase between the MFMAs of another.
@@ -67,6 +66,8 @@ __host__ __device__ constexpr int odd_axes(int k) { return (k & 1) + ((k >> 1) &
 template <int P>
 struct Cls {
     static constexpr int HE = (P + 1) / 2, HO = P / 2;  // even / odd half-nodes per axis
+    static constexpr int kH3 = HE * HE * HE;
+    static constexpr int kItems = (kH3 * 16 + kMThreads - 1) / kMThreads;  // half-nodes of 16 cells per thread
     __host__ __device__ static constexpr int side(int k, int a) { return (k >> a) & 1 ? HO : HE; }
     // half-nodes of a class with o odd axes, MFMA K steps (4 half-nodes), row tiles (16)
     __host__ __device__ static constexpr int size(int o) {
@@ -102,24 +103,23 @@ struct Cls {
     }
 };
 
-// One row of the products: its offset |pos|, the rows of the offset's segment
-// in the row block, and its place in a target's C (variant 0).
-struct RowInfo {
-    uint16_t tau, seg;
-    int32_t off;
+// One row of the products: its offset |pos|, its place in a target's C (bytes,
+// variant 0), and the bytes that a negative sign of each coordinate adds (0:
+// only one sign, or none, belongs to the offset).
+struct __attribute__((aligned(16))) RowInfo {
+    uint32_t tau, off;
+    uint16_t sign[3], pad;
 };
 
 struct M2LArgs {
     M2LLevels lv;
     int64_t first, ncell;  // cells of the working levels
     int rb0, rb1;          // row blocks of this launch
-    int off0, stride;      // C offset of rb0, and C doubles per target
+    uint32_t off0, stride;  // C bytes before rb0, and C bytes per target
     const int32_t* slots;
     const uint64_t* keys;
     const RowInfo* rows;
-    const uint8_t* vtab;       // [57][8] variant of (offset, sigma), kNoSlot: none
-    const uint8_t* jmap;       // [8][57][8] slot of the target that a source of a parity has at (offset, sigma)
-    const uint16_t* slot_tau;  // [8][189] 8 offset + sigma of a target's slot
+    const uint16_t* slot_tau;  // [8][189] 8 offset + sigma of a target's slot, then the same seen from the other cell
     const double* ops;         // fragments, row block by row block
     double* C;
     double* acc;               // partial locals between launches over parts of the rows
@@ -153,8 +153,8 @@ __device__ __forceinline__ void hadamard8(double (&d)[8]) {
 // store is dropped and a load gives 0, so a lane without a partner takes part
 // with the offset kNowhere.  A branch around each access would hide their number
 // from the wait counts: every wait for operators would wait for all stores.
-constexpr uint32_t kNowhere = 0xFFFFFFF8u;
-constexpr size_t kBufferMax = 0xFFFF0000u;  // bytes
+constexpr uint32_t kNowhere = 0xFFF00000u;  // plus an offset in a target's C (below 1 MiB)
+constexpr size_t kBufferMax = kNowhere;     // bytes
 
 typedef uint32_t u2 __attribute__((ext_vector_type(2)));
 
@@ -168,10 +168,20 @@ __device__ __forceinline__ void buffer_store(__amdgpu_buffer_rsrc_t r, uint32_t 
     __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v), r, static_cast<int>(off), 0, 0);
 }
 
+// Bytes into a target's C of the 8 signs of a row.
+__device__ __forceinline__ void variant_offsets(const RowInfo& r, uint32_t off0, uint32_t (&at)[8]) {
+    at[0] = r.off - off0;
+    at[1] = at[0] + r.sign[0];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) at[2 + s] = at[s] + r.sign[1];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) at[4 + s] = at[s] + r.sign[2];
+}
+
 // The steps (RB row blocks each) of [rb0, rb1) that hold a flagged offset, in
 // ascending order, as step numbers relative to rb0; called by every thread.
 template <int RB>
-__device__ __forceinline__ int active_steps(const M2LArgs& a, const RowInfo* s_rows, const int* s_flag, uint16_t* s_list,
+__device__ __forceinline__ int active_steps(const M2LArgs& a, const int* s_flag, uint16_t* s_list,
                                             int* s_count) {
     const int nst = (a.rb1 - a.rb0 + RB - 1) / RB;
     if (threadIdx.x < 64) {
@@ -180,9 +190,10 @@ __device__ __forceinline__ int active_steps(const M2LArgs& a, const RowInfo* s_r
             const int st = b + static_cast<int>(threadIdx.x);
             bool on = false;
             if (st < nst) {
-                const int r0 = 16 * RB * st;
-                const int r1 = min(r0 + 16 * RB, 16 * (a.rb1 - a.rb0)) - 1;
-                for (int t = s_rows[r0].tau; t <= s_rows[r1].tau; ++t) on |= s_flag[t] != 0;
+                const int r0 = 16 * (a.rb0 + RB * st);
+                const int r1 = min(r0 + 16 * RB, 16 * a.rb1) - 1;
+                const int t0 = a.rows[r0].tau, t1 = a.rows[r1].tau;
+                for (int t = t0; t <= t1; ++t) on |= s_flag[t] != 0;
             }
             const uint64_t m = __ballot(on);
             if (on) s_list[n + __popcll(m & ((1ull << threadIdx.x) - 1ull))] = static_cast<uint16_t>(st);
@@ -203,30 +214,26 @@ struct Lds {
 };
 
 struct SmemLayout {
-    int rows, tabs, cells, flags, bytes;  // byte offsets
+    int cells, rows, flags, bytes;  // byte offsets
 };
-inline SmemLayout smem_layout(int big_doubles, int nrows, int tab_bytes, int cell_bytes) {
+inline SmemLayout smem_layout(int big_doubles, int cell_bytes, int nrows) {
     SmemLayout s;
-    s.rows = big_doubles * 8;
-    s.tabs = s.rows + nrows * static_cast<int>(sizeof(RowInfo));
-    s.cells = s.tabs + ((tab_bytes + 15) & ~15);
-    s.flags = s.cells + ((cell_bytes + 15) & ~15);
+    s.cells = big_doubles * 8;
+    s.rows = s.cells + ((cell_bytes + 15) & ~15);
+    s.flags = s.rows + nrows * static_cast<int>(sizeof(RowInfo));
     s.bytes = s.flags + 4 * (kTau + 2 + 2) + 2 * kMaxSteps;
     return s;
 }
 
 // ---------------------------------------------------------------------------
 template <int P, int C, int O, bool WIDE>
-__device__ __forceinline__ void up_body(const M2LArgs& a, const SmemLayout& sl, char* smem, const double* __restrict__ M,
-                                        int LD, int wave, int64_t cell0, int ncol) {
+__device__ __forceinline__ void up_body(const M2LArgs& a, const SmemLayout& sl, char* smem,
+                                        double (&nodes)[C][Cls<P>::kItems][8], int wave) {
     using K = Cls<P>;
     constexpr int RB = Lds<C>::RB, KROW = Lds<C>::kRow, BUF = Lds<C>::kBuf;
     constexpr int KS = K::ks(O), KSP = K::ksp(O);
     double* big = reinterpret_cast<double*>(smem);
-    const RowInfo* s_rows = reinterpret_cast<const RowInfo*>(smem + sl.rows);
-    const uint8_t* s_vtab = reinterpret_cast<const uint8_t*>(smem + sl.tabs);
-    const uint8_t* s_jmap = s_vtab + 8 * (kTau + 1);
-    const int32_t* s_tgt = reinterpret_cast<const int32_t*>(smem + sl.cells);
+    const uint32_t* s_tgt = reinterpret_cast<const uint32_t*>(smem + sl.cells);
     int* s_flag = reinterpret_cast<int*>(smem + sl.flags);
     int* s_count = s_flag + kTau + 2;
     uint16_t* s_list = reinterpret_cast<uint16_t*>(s_flag + kTau + 4);
@@ -236,19 +243,13 @@ __device__ __forceinline__ void up_body(const M2LArgs& a, const SmemLayout& sl, 
     double b[C][KS];
 #pragma unroll
     for (int c = 0; c < C; ++c) {
-        for (int e = tid; e < K::HE * K::HE * K::HE * 16; e += kMThreads) {
-            const int h = e % (K::HE * K::HE * K::HE), cc = e / (K::HE * K::HE * K::HE);
-            const int hx = h % K::HE, hy = (h / K::HE) % K::HE, hz = h / (K::HE * K::HE);
-            const int64_t cell = cell0 + 16 * c + cc;
-            const bool in = 16 * c + cc < ncol;
-            double d[8];
 #pragma unroll
-            for (int f = 0; f < 8; ++f) {
-                // a middle node (odd order) has no mirror image
-                const bool mid = ((f & 1) && hx == K::HO) || ((f & 2) && hy == K::HO) || ((f & 4) && hz == K::HO);
-                const int nx = f & 1 ? P - 1 - hx : hx, ny = f & 2 ? P - 1 - hy : hy, nz = f & 4 ? P - 1 - hz : hz;
-                d[f] = (in && !mid) ? M[cell * LD + (nz * P + ny) * P + nx] : 0.;
-            }
+        for (int it = 0; it < K::kItems; ++it) {
+            const int e = tid + it * kMThreads;
+            if (K::kH3 * 16 % kMThreads && e >= K::kH3 * 16) break;
+            const int h = e % K::kH3, cc = e / K::kH3;
+            const int hx = h % K::HE, hy = (h / K::HE) % K::HE, hz = h / (K::HE * K::HE);
+            double(&d)[8] = nodes[c][it];
             hadamard8(d);
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
@@ -274,7 +275,7 @@ __device__ __forceinline__ void up_body(const M2LArgs& a, const SmemLayout& sl, 
         for (int s = 0; s < KS; ++s) b[c][s] = mine[off + 64 * s];
         __syncthreads();
     }
-    const int nact = active_steps<RB>(a, s_rows, s_flag, s_list, s_count);
+    const int nact = active_steps<RB>(a, s_flag, s_list, s_count);
     if (nact == 0) return;
 
     int wop = 0, rbd = 0;
@@ -287,10 +288,8 @@ __device__ __forceinline__ void up_body(const M2LArgs& a, const SmemLayout& sl, 
     const double2* ops = reinterpret_cast<const double2*>(a.ops + static_cast<int64_t>(a.rb0) * rbd + wop) + lane;
     // this thread's line of a step's Hadamard sums
     const int erow = tid % (16 * RB), ecol = tid / (16 * RB);
-    const int epar = ecol < ncol ? static_cast<int>(a.keys[cell0 + ecol] & 7u) : 0;
-    const uint8_t* ejm = s_jmap + epar * 8 * (kTau + 1);
-    const int32_t* etg = s_tgt + ecol * kTgtRow;
-    const __amdgpu_buffer_rsrc_t out = buffer_of(a.C, static_cast<uint32_t>(8 * a.stride * a.ncell));
+    const uint32_t* etg = s_tgt + ecol * kTgtRow;
+    const __amdgpu_buffer_rsrc_t out = buffer_of(a.C, static_cast<uint32_t>(a.stride * a.ncell));
 
     auto fetch = [&](int st, double2 (&o)[RB][KSP]) {
 #pragma unroll
@@ -328,32 +327,31 @@ __device__ __forceinline__ void up_body(const M2LArgs& a, const SmemLayout& sl, 
     };
     // the sums of a step in three parts, between the MFMAs of the next
     double d[8];
+    const RowInfo* rows = reinterpret_cast<const RowInfo*>(smem + sl.rows) + erow;
     RowInfo ri;
-    int tg[8];
-    uint64_t vt;
+    uint32_t tg[8];
     auto send_read = [&](int buf, int st) {
-        ri = s_rows[16 * RB * st + erow];
+        ri = rows[16 * RB * st];
 #pragma unroll
         for (int k = 0; k < 8; ++k) d[k] = big[buf * BUF + (wave_of(k) * 16 * C + ecol) * KROW + erow];
     };
     auto send_sum = [&]() {
-        const uint64_t jm = *reinterpret_cast<const uint64_t*>(ejm + 8 * ri.tau);
-        vt = *reinterpret_cast<const uint64_t*>(s_vtab + 8 * ri.tau);
-#pragma unroll
-        for (int s = 0; s < 8; ++s) {
-            const int j = static_cast<int>((jm >> (8 * s)) & 255u);
-            tg[s] = etg[j];  // kNoSlot: a slot past the cell's own that holds none
-        }
+        const uint4* t = reinterpret_cast<const uint4*>(etg + 8 * ri.tau);
+        const uint4 lo = t[0], hi = t[1];
+        tg[0] = lo.x, tg[1] = lo.y, tg[2] = lo.z, tg[3] = lo.w;
+        tg[4] = hi.x, tg[5] = hi.y, tg[6] = hi.z, tg[7] = hi.w;
         hadamard8(d);
     };
     auto send_store = [&]() {
+        uint32_t at[8];
+        variant_offsets(ri, a.off0, at);
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
-            const int at = ri.off - a.off0 + static_cast<int>((vt >> (8 * s)) & 255u) * ri.seg;
-            if constexpr (WIDE) {
-                if (tg[s] >= 0) a.C[static_cast<int64_t>(tg[s]) * a.stride + at] = d[s];
+            if constexpr (WIDE) {  // tg: the target itself
+                if (tg[s] != kNowhere)
+                    *reinterpret_cast<double*>(reinterpret_cast<char*>(a.C) + static_cast<uint64_t>(tg[s]) * a.stride + at[s]) = d[s];
             } else {
-                buffer_store(out, tg[s] >= 0 ? 8u * (static_cast<uint32_t>(tg[s]) * a.stride + at) : kNowhere, d[s]);
+                buffer_store(out, tg[s] + at[s], d[s]);
             }
         }
     };
@@ -399,16 +397,59 @@ __device__ __forceinline__ void up_body(const M2LArgs& a, const SmemLayout& sl, 
     send_store();
 }
 
-// Rows, tables and the per-cell slots of a tile into the LDS; flags the
-// offsets that any cell of the tile interacts at.
-__device__ __forceinline__ void load_rows(const M2LArgs& a, const SmemLayout& sl, char* smem) {
-    uint64_t* r = reinterpret_cast<uint64_t*>(smem + sl.rows);
-    const uint64_t* g = reinterpret_cast<const uint64_t*>(a.rows + 16 * static_cast<int64_t>(a.rb0));
-    for (int i = threadIdx.x; i < 16 * (a.rb1 - a.rb0); i += kMThreads) r[i] = g[i];
-    uint64_t* v = reinterpret_cast<uint64_t*>(smem + sl.tabs);
-    for (int i = threadIdx.x; i < kTau + 1; i += kMThreads) v[i] = reinterpret_cast<const uint64_t*>(a.vtab)[i];
-    int* s_flag = reinterpret_cast<int*>(smem + sl.flags);
-    if (threadIdx.x < kTau + 2) s_flag[threadIdx.x] = 0;
+// The slots of a tile's cells, kSlotItems per thread (the cells' rows are
+// contiguous), -1 past the last cell.
+template <int C>
+struct TileSlots {
+    static constexpr int kSlotItems = (16 * C * kFarSlots + kMThreads - 1) / kMThreads;
+    int32_t t[kSlotItems];
+    __device__ __forceinline__ void load(const M2LArgs& a, int64_t cell0, int ncol) {
+        const int32_t* g = a.slots + cell0 * kFarSlots;
+#pragma unroll
+        for (int i = 0; i < kSlotItems; ++i) {
+            const int e = static_cast<int>(threadIdx.x) + i * kMThreads;
+            t[i] = e < ncol * kFarSlots ? g[e] : -1;
+        }
+    }
+    // f(cell of the tile, 8 offset + sigma, slot value) for every slot that is taken
+    template <class F>
+    __device__ __forceinline__ void each(const uint16_t* s_slot, const int* s_par, F f) const {
+#pragma unroll
+        for (int i = 0; i < kSlotItems; ++i) {
+            if (t[i] < 0) continue;
+            const int e = static_cast<int>(threadIdx.x) + i * kMThreads;
+            const int cc = e / kFarSlots, j = e - cc * kFarSlots;
+            f(cc, static_cast<int>(s_slot[s_par[cc] * kFarSlots + j]), t[i]);
+        }
+    }
+};
+
+// The slots' table (dir 0: positions seen from the cell, 1:
+// from the other cell), the parities and the
+// first cells of the levels of the tile's cells into the LDS.
+struct TileTables {
+    uint16_t* slot;  // at the end of the tile buffers, free before the first step
+    int* par;
+    int* first;
+    int* flag;
+};
+template <int C>
+__device__ __forceinline__ TileTables load_tables(const M2LArgs& a, const SmemLayout& sl, char* smem, int dir, int64_t cell0,
+                                                  int ncol) {
+    TileTables t;
+    t.slot = reinterpret_cast<uint16_t*>(smem + sl.cells) - 8 * kFarSlots;
+    t.par = reinterpret_cast<int*>(t.slot) - 32;
+    t.first = t.par - 32;
+    t.flag = reinterpret_cast<int*>(smem + sl.flags);
+    const uint32_t* st = reinterpret_cast<const uint32_t*>(a.slot_tau + dir * 8 * kFarSlots);
+    for (int i = threadIdx.x; i < 4 * kFarSlots; i += kMThreads) reinterpret_cast<uint32_t*>(t.slot)[i] = st[i];
+    if (threadIdx.x < kTau + 2) t.flag[threadIdx.x] = 0;
+    if (static_cast<int>(threadIdx.x) < ncol) {
+        const int64_t cell = cell0 + threadIdx.x;
+        t.par[threadIdx.x] = static_cast<int>(a.keys[cell] & 7u);
+        t.first[threadIdx.x] = static_cast<int>(a.lv.cell_off[level_of(a.lv, cell)] - a.first);
+    }
+    return t;
 }
 
 template <int P, int C, bool WIDE>
@@ -419,34 +460,52 @@ __global__ __launch_bounds__(kMThreads, 2) void k_m2l_up(M2LArgs a, SmemLayout s
     const int64_t end = a.first + a.ncell;
     if (cell0 >= end) return;  // the same for the whole workgroup
     const int ncol = static_cast<int>(min(static_cast<int64_t>(16 * C), end - cell0));
-    load_rows(a, sl, smem);
-    uint64_t* s_jmap = reinterpret_cast<uint64_t*>(smem + sl.tabs) + kTau + 1;
-    for (int i = threadIdx.x; i < 8 * (kTau + 1); i += kMThreads) s_jmap[i] = reinterpret_cast<const uint64_t*>(a.jmap)[i];
-    int32_t* s_tgt = reinterpret_cast<int32_t*>(smem + sl.cells);
-    int* s_flag = reinterpret_cast<int*>(smem + sl.flags);
-    __syncthreads();
-    for (int e = threadIdx.x; e < 16 * C * kTgtRow; e += kMThreads) {
-        const int cc = e / kTgtRow, j = e % kTgtRow;
-        int t = -1;
-        if (cc < ncol && j < kFarSlots) {
-            const int64_t cell = cell0 + cc;
-            t = a.slots[cell * kFarSlots + j];
-            if (t >= 0) {
-                t = static_cast<int>(a.lv.cell_off[level_of(a.lv, cell)] + t - a.first);
-                s_flag[a.slot_tau[static_cast<int>(a.keys[cell] & 7u) * kFarSlots + j] >> 3] = 1;
+    // every load of the prologue on its way at once
+    using K = Cls<P>;
+    TileSlots<C> ts;
+    ts.load(a, cell0, ncol);
+    double nodes[C][K::kItems][8];
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+#pragma unroll
+        for (int it = 0; it < K::kItems; ++it) {
+            const int e = static_cast<int>(threadIdx.x) + it * kMThreads;
+            const int h = e % K::kH3, cc = 16 * c + e / K::kH3;
+            const int hx = h % K::HE, hy = (h / K::HE) % K::HE, hz = h / (K::HE * K::HE);
+            const bool in = cc < ncol && e < K::kH3 * 16;
+            const double* m = M + (cell0 + (in ? cc : 0)) * LD;
+#pragma unroll
+            for (int f = 0; f < 8; ++f) {
+                // a middle node (odd order) has no mirror image
+                const bool mid = ((f & 1) && hx == K::HO) || ((f & 2) && hy == K::HO) || ((f & 4) && hz == K::HO);
+                const int nx = f & 1 ? P - 1 - hx : hx, ny = f & 2 ? P - 1 - hy : hy, nz = f & 4 ? P - 1 - hz : hz;
+                const double v = m[(nz * P + ny) * P + nx];
+                nodes[c][it][f] = in && !mid ? v : 0.;
             }
         }
-        s_tgt[e] = t;
-    }
+    const TileTables tt = load_tables<C>(a, sl, smem, 1, cell0, ncol);
+    for (int i = threadIdx.x; i < 16 * (a.rb1 - a.rb0); i += kMThreads)
+        reinterpret_cast<uint4*>(smem + sl.rows)[i] = reinterpret_cast<const uint4*>(a.rows + 16 * static_cast<int64_t>(a.rb0))[i];
+    // targets of every source by (offset, sigma): where their C begins
+    uint32_t* s_tgt = reinterpret_cast<uint32_t*>(smem + sl.cells);
+    for (int e = threadIdx.x; e < 4 * C * kTgtRow; e += kMThreads)
+        reinterpret_cast<uint4*>(s_tgt)[e] = make_uint4(kNowhere, kNowhere, kNowhere, kNowhere);
+    __syncthreads();
+    ts.each(tt.slot, tt.par, [&](int cc, int w, int t) {
+        const uint32_t to = static_cast<uint32_t>(tt.first[cc] + t);
+        s_tgt[cc * kTgtRow + w] = WIDE ? to : to * a.stride;
+        tt.flag[w >> 3] = 1;
+    });
+    __syncthreads();
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if constexpr (P % 2 == 0) {
-        up_body<P, C, 0, WIDE>(a, sl, smem, M, LD, wave, cell0, ncol);
+        up_body<P, C, 0, WIDE>(a, sl, smem, nodes, wave);
     } else {
         switch (odd_axes(class_of(wave))) {
-            case 0: up_body<P, C, 0, WIDE>(a, sl, smem, M, LD, wave, cell0, ncol); break;
-            case 1: up_body<P, C, 1, WIDE>(a, sl, smem, M, LD, wave, cell0, ncol); break;
-            case 2: up_body<P, C, 2, WIDE>(a, sl, smem, M, LD, wave, cell0, ncol); break;
-            default: up_body<P, C, 3, WIDE>(a, sl, smem, M, LD, wave, cell0, ncol); break;
+            case 0: up_body<P, C, 0, WIDE>(a, sl, smem, nodes, wave); break;
+            case 1: up_body<P, C, 1, WIDE>(a, sl, smem, nodes, wave); break;
+            case 2: up_body<P, C, 2, WIDE>(a, sl, smem, nodes, wave); break;
+            default: up_body<P, C, 3, WIDE>(a, sl, smem, nodes, wave); break;
         }
     }
 }
@@ -459,14 +518,12 @@ __device__ __forceinline__ void down_body(const M2LArgs& a, const SmemLayout& sl
     constexpr int RB = Lds<C>::RB, KROW = Lds<C>::kRow, BUF = Lds<C>::kBuf;
     constexpr int NT = K::nt(O);
     double* big = reinterpret_cast<double*>(smem);
-    const RowInfo* s_rows = reinterpret_cast<const RowInfo*>(smem + sl.rows);
-    const uint8_t* s_vtab = reinterpret_cast<const uint8_t*>(smem + sl.tabs);
     const uint8_t* s_ex = reinterpret_cast<const uint8_t*>(smem + sl.cells);
     int* s_flag = reinterpret_cast<int*>(smem + sl.flags);
     int* s_count = s_flag + kTau + 2;
     uint16_t* s_list = reinterpret_cast<uint16_t*>(s_flag + kTau + 4);
     const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, kq = lane >> 4;
-    const int nact = active_steps<RB>(a, s_rows, s_flag, s_list, s_count);
+    const int nact = active_steps<RB>(a, s_flag, s_list, s_count);
 
     int wop = 0, rbd = 0, lrow = 0;
 #pragma unroll
@@ -486,16 +543,16 @@ __device__ __forceinline__ void down_body(const M2LArgs& a, const SmemLayout& sl
     const int erow = tid % (16 * RB), ecol = tid / (16 * RB);
     // the C of the tile's targets
     const __amdgpu_buffer_rsrc_t in =
-        buffer_of(a.C + (cell0 - a.first) * a.stride, static_cast<uint32_t>(8 * a.stride * ncol));
-    const int mine = ecol * a.stride - a.off0;
-    auto fetch = [&](int st, double (&d)[8]) {
-        const RowInfo ri = s_rows[16 * RB * st + erow];
-        const int ex = s_ex[ecol * kTauStride + ri.tau];
-        const uint64_t vt = *reinterpret_cast<const uint64_t*>(s_vtab + 8 * ri.tau);
+        buffer_of(reinterpret_cast<double*>(reinterpret_cast<char*>(a.C) + (cell0 - a.first) * a.stride), a.stride * ncol);
+    const uint32_t mine = a.off0 - ecol * a.stride;
+    const RowInfo* rows = a.rows + 16 * a.rb0 + erow;
+    auto fetch = [&](const RowInfo& ri, double (&d)[8]) {
+        const int none = ~static_cast<int>(s_ex[ecol * kTauStride + ri.tau]);
+        uint32_t at[8];
+        variant_offsets(ri, mine, at);
 #pragma unroll
-        for (int s = 0; s < 8; ++s)
-            d[s] = buffer_load(in, (ex >> s) & 1 ? 8u * (mine + ri.off + static_cast<int>((vt >> (8 * s)) & 255u) * ri.seg)
-                                                 : kNowhere);
+        for (int s = 0; s < 8; ++s)  // past every end, where there is no source
+            d[s] = buffer_load(in, at[s] | (static_cast<uint32_t>(__builtin_amdgcn_sbfe(none, s, 1)) & 0xFFFFFFF0u));
     };
     auto sums = [&](int buf, double (&d)[8]) {
         hadamard8(d);
@@ -512,6 +569,7 @@ __device__ __forceinline__ void down_body(const M2LArgs& a, const SmemLayout& sl
     };
     // operators of the next step and C of the one after it on their way during
     // this step's products, the next step's sums between them
+    RowInfo rn;  // of the next C to fetch
     auto step = [&](int i, const double2 (&av)[RB][NT][2], double2 (&nv)[RB][NT][2], double (&d)[8]) {
         double2 bv[RB][C][2];
 #pragma unroll
@@ -542,7 +600,8 @@ __device__ __forceinline__ void down_body(const M2LArgs& a, const SmemLayout& sl
         M2L_FENCE;
         products(1);
         M2L_FENCE;
-        fetch(s_list[i + 2 < nact ? i + 2 : i], d);
+        fetch(rn, d);
+        rn = rows[16 * RB * s_list[i + 3 < nact ? i + 3 : i]];
         M2L_FENCE;
         products(2);
         products(3);
@@ -551,10 +610,13 @@ __device__ __forceinline__ void down_body(const M2LArgs& a, const SmemLayout& sl
     if (nact > 0) {
         double d[8];
         double2 ev[RB][NT][2], ov[RB][NT][2];
-        fetch(s_list[0], d);
+        rn = rows[16 * RB * s_list[0]];
+        fetch(rn, d);
         operators(s_list[0], ev);
+        rn = rows[16 * RB * s_list[nact > 1 ? 1 : 0]];
         sums(0, d);
-        fetch(s_list[nact > 1 ? 1 : 0], d);
+        fetch(rn, d);
+        rn = rows[16 * RB * s_list[nact > 2 ? 2 : 0]];
         __syncthreads();
         int i = 0;
         for (; i + 1 < nact; i += 2) {
@@ -571,7 +633,6 @@ __device__ __forceinline__ void down_body(const M2LArgs& a, const SmemLayout& sl
         return;
     }
     // the classes back to nodes, one column tile at a time
-    constexpr int H3 = K::HE * K::HE * K::HE;
 #pragma unroll
     for (int c = 0; c < C; ++c) {
         if (c) __syncthreads();
@@ -580,8 +641,8 @@ __device__ __forceinline__ void down_body(const M2LArgs& a, const SmemLayout& sl
 #pragma unroll
             for (int r = 0; r < 4; ++r) big[(lrow + 16 * t + 4 * r + kq) * 17 + col] = acc[t][c][r];
         __syncthreads();
-        for (int e = tid; e < H3 * 16; e += kMThreads) {
-            const int h = e % H3, cc = e / H3;
+        for (int e = tid; e < K::kH3 * 16; e += kMThreads) {
+            const int h = e % K::kH3, cc = e / K::kH3;
             if (16 * c + cc >= ncol) continue;
             const int hx = h % K::HE, hy = (h / K::HE) % K::HE, hz = h / (K::HE * K::HE);
             double d[8];
@@ -615,20 +676,22 @@ __global__ __launch_bounds__(kMThreads, 2) void k_m2l_down(M2LArgs a, SmemLayout
     const int64_t end = a.first + a.ncell;
     if (cell0 >= end) return;
     const int ncol = static_cast<int>(min(static_cast<int64_t>(16 * C), end - cell0));
-    load_rows(a, sl, smem);
-    uint32_t* s_ex = reinterpret_cast<uint32_t*>(smem + sl.cells);
-    for (int i = threadIdx.x; i < 16 * C * kTauStride / 4; i += kMThreads) s_ex[i] = 0u;
-    int* s_flag = reinterpret_cast<int*>(smem + sl.flags);
+    TileSlots<C> ts;
+    ts.load(a, cell0, ncol);
+    const TileTables tt = load_tables<C>(a, sl, smem, 0, cell0, ncol);
+    // signs of each offset that a target has a source at: a byte per (target,
+    // offset, sigma) in the tile buffers, then packed to a bit each
+    uint64_t* s_at = reinterpret_cast<uint64_t*>(smem);
+    for (int i = threadIdx.x; i < 16 * C * kTauStride; i += kMThreads) s_at[i] = 0ull;
     __syncthreads();
-    for (int e = threadIdx.x; e < ncol * kFarSlots; e += kMThreads) {
-        const int cc = e / kFarSlots, j = e % kFarSlots;
-        const int64_t cell = cell0 + cc;
-        if (a.slots[cell * kFarSlots + j] < 0) continue;
-        const int ts = a.slot_tau[static_cast<int>(a.keys[cell] & 7u) * kFarSlots + j];
-        const int byte = cc * kTauStride + (ts >> 3);
-        atomicOr(&s_ex[byte >> 2], 1u << (8 * (byte & 3) + (ts & 7)));
-        s_flag[ts >> 3] = 1;
-    }
+    ts.each(tt.slot, tt.par, [&](int cc, int w, int) {
+        reinterpret_cast<uint8_t*>(s_at)[cc * 8 * kTauStride + w] = 1;
+        tt.flag[w >> 3] = 1;
+    });
+    __syncthreads();
+    uint8_t* s_ex = reinterpret_cast<uint8_t*>(smem + sl.cells);
+    for (int i = threadIdx.x; i < 16 * C * kTauStride; i += kMThreads)
+        s_ex[i] = static_cast<uint8_t>((s_at[i] * 0x0102040810204080ull) >> 56);  // byte k (0 or 1) -> bit k
     __syncthreads();
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if constexpr (P % 2 == 0) {
@@ -719,8 +782,6 @@ __global__ __launch_bounds__(256) void k_m2l_pack(const RowInfo* __restrict__ ro
     }
 }
 
-constexpr int kVtabBytes = 8 * (kTau + 1), kJmapBytes = 8 * kVtabBytes, kSlotTauBytes = 2 * 8 * kFarSlots;
-
 template <int P>
 int pack_impl(Context* c, int nrb, const TauInfo* tau) {
     using K = Cls<P>;
@@ -739,6 +800,7 @@ int pack_impl(Context* c, int nrb, const TauInfo* tau) {
 // parts, whose partial locals pass through memory (p^3 doubles per cell and
 // part).  Where one step's C is larger still (more than 4 million cells),
 // addresses take 64 bits.
+constexpr int kMaxPart = 116;  // row blocks of a launch: their table fits the LDS beside the tiles
 constexpr int64_t kTwoTiles = 16 * 1024;  // cells from which a workgroup takes two column tiles
 
 template <int P, int C, bool WIDE>
@@ -754,12 +816,13 @@ int m2l_launch(Context* c, M2LArgs a) {
     while (cut.back() < nrb) {
         int e = cut.back() + RB;
         auto width = [&](int to) { return c->m2l_rboff[to] - c->m2l_rboff[cut.back()]; };
-        while (e < nrb && sizeof(double) * static_cast<size_t>(width(std::min(e + RB, nrb))) * a.ncell <= kBufferMax) e += RB;
+        while (e < nrb && e + RB - cut.back() <= kMaxPart &&
+               static_cast<size_t>(width(std::min(e + RB, nrb))) * a.ncell <= kBufferMax) e += RB;
         e = std::min(e, nrb);
         stride = std::max<int64_t>(stride, width(e));
         cut.push_back(e);
     }
-    HFMM_TRY(ensure(c, c->d_m2lC, sizeof(double) * static_cast<size_t>(stride) * a.ncell));
+    HFMM_TRY(ensure(c, c->d_m2lC, static_cast<size_t>(stride) * a.ncell));
     a.C = c->d_m2lC.as<double>();
     const int parts = static_cast<int>(cut.size()) - 1;
     if (parts > 1)
@@ -768,9 +831,8 @@ int m2l_launch(Context* c, M2LArgs a) {
     int maxrows = 0;
     for (int i = 0; i < parts; ++i) maxrows = std::max(maxrows, 16 * (cut[i + 1] - cut[i]));
     const int tilebuf = 2 * Lds<C>::kBuf;
-    const SmemLayout su = smem_layout(std::max(tilebuf, K::exp_off(8)), maxrows, kVtabBytes + kJmapBytes,
-                                      16 * C * kTgtRow * 4);
-    const SmemLayout sd = smem_layout(std::max(tilebuf, 17 * K::loc_off(8)), maxrows, kVtabBytes, 16 * C * kTauStride);
+    const SmemLayout su = smem_layout(std::max(tilebuf, K::exp_off(8)), 16 * C * kTgtRow * 4, maxrows);
+    const SmemLayout sd = smem_layout(std::max(tilebuf, 17 * K::loc_off(8)), 16 * C * kTauStride, 0);
     static int lds_up[64] = {0}, lds_down[64] = {0};
     HFMM_TRY(raise_lds_limit(c, reinterpret_cast<const void*>(&k_m2l_up<P, C, WIDE>), su.bytes, lds_up));
     HFMM_TRY(raise_lds_limit(c, reinterpret_cast<const void*>(&k_m2l_down<P, C>), sd.bytes, lds_down));
@@ -810,13 +872,10 @@ int m2l_impl(Context* c) {
     a.slots = c->d_m2l.as<int32_t>();
     a.keys = c->d_cellkey.as<uint64_t>();
     a.rows = c->d_m2lrows.as<RowInfo>();
-    const uint8_t* t = c->d_m2ltab.as<uint8_t>();
-    a.vtab = t;
-    a.jmap = t + kVtabBytes;
-    a.slot_tau = reinterpret_cast<const uint16_t*>(t + kVtabBytes + kJmapBytes);
+    a.slot_tau = c->d_m2ltab.as<uint16_t>();
     int step = 0;
     for (int b = 0; b < c->m2l_nrb; ++b) step = std::max(step, c->m2l_rboff[b + 1] - c->m2l_rboff[b]);
-    if (sizeof(double) * static_cast<size_t>(step) * a.ncell > kBufferMax) return m2l_launch<P, 2, true>(c, a);
+    if (static_cast<size_t>(step) * a.ncell > kBufferMax) return m2l_launch<P, 2, true>(c, a);
     return a.ncell >= kTwoTiles ? m2l_launch<P, 2, false>(c, a) : m2l_launch<P, 1, false>(c, a);
 }
 
@@ -852,30 +911,7 @@ int prepare_m2l_f64(Context* c) {
             }
     const int nrb = ((row + 15) / 16 + 1) & ~1;  // whole steps of either tile shape
     if (n != kTau || nrb > kMaxSteps) return fail(c, HFMM_ERR_ARG, "operator rank above 64 is not supported");
-    // variants: one bit per axis whose both signs occur for a target (|x| = 3 has one, by its parity)
-    std::vector<uint8_t> tab(kVtabBytes + kJmapBytes + kSlotTauBytes, static_cast<uint8_t>(kNoSlot));
-    int nvar[kTau];
-    for (int x = 0; x < 4; ++x)
-        for (int y = 0; y < 4; ++y)
-            for (int z = 0; z < 4; ++z) {
-                const int t = tau_of[x][y][z];
-                if (t < 0) continue;
-                const int v[3] = {x, y, z};
-                nvar[t] = 1;
-                for (int a = 0; a < 3; ++a) nvar[t] *= v[a] == 1 || v[a] == 2 ? 2 : 1;
-                for (int s = 0; s < 8; ++s) {
-                    int idx = 0, bit = 0;
-                    bool ok = true;
-                    for (int a = 0; a < 3; ++a) {
-                        const int sb = (s >> a) & 1;
-                        if (v[a] == 0) ok &= sb == 0;
-                        else if (v[a] < 3) idx |= sb << bit++;
-                    }
-                    if (ok) tab[8 * t + s] = static_cast<uint8_t>(idx);
-                }
-            }
-    uint8_t* jmap = tab.data() + kVtabBytes;
-    uint16_t* slot_tau = reinterpret_cast<uint16_t*>(tab.data() + kVtabBytes + kJmapBytes);
+    std::vector<uint16_t> slot_tau(2 * 8 * kFarSlots);
     for (int e = 0; e < 8; ++e) {
         FarSlot fs[kFarSlots];
         far_slots(e, fs);
@@ -888,26 +924,36 @@ int prepare_m2l_f64(Context* c) {
                 if (d[a] > 0) back |= 1 << a;
             }
             slot_tau[e * kFarSlots + j] = static_cast<uint16_t>(8 * t + s);
-            jmap[(e * (kTau + 1) + t) * 8 + back] = static_cast<uint8_t>(j);
+            slot_tau[(8 + e) * kFarSlots + j] = static_cast<uint16_t>(8 * t + back);
         }
     }
-    // a target's C: row block by row block, in it per offset [variant][rows of the offset in the block]
-    std::vector<RowInfo> rows(static_cast<size_t>(nrb) * 16, RowInfo{kTauDummy, 0, 0});
+    // a target's C: row block by row block, in it per offset [variant][rows of
+    // the offset in the block]; a variant per pair of signs that a target of
+    // one parity has on an axis (|x| = 1, 2: both; 3: one, by its parity; 0: none)
+    std::vector<RowInfo> rows(static_cast<size_t>(nrb) * 16, RowInfo{kTauDummy, 0, {0, 0, 0}, 0});
     for (int t = 0; t < kTau; ++t)
-        for (int r = 0; r < ((tau[t].rank + 3) & ~3); ++r) rows[tau[t].row0 + r].tau = static_cast<uint16_t>(t);
+        for (int r = 0; r < ((tau[t].rank + 3) & ~3); ++r) rows[tau[t].row0 + r].tau = static_cast<uint32_t>(t);
     c->m2l_rboff.assign(nrb + 1, 0);
     int off = 0;
     for (int b = 0; b < nrb; ++b) {
         c->m2l_rboff[b] = off;
         for (int r = 0; r < 16;) {
-            const int t = rows[16 * b + r].tau;
+            const int t = static_cast<int>(rows[16 * b + r].tau);
             int e = r;
-            while (e < 16 && rows[16 * b + e].tau == t) ++e;
-            for (int q = r; q < e; ++q) {
-                rows[16 * b + q].seg = static_cast<uint16_t>(e - r);
-                rows[16 * b + q].off = off + q - r;
+            while (e < 16 && static_cast<int>(rows[16 * b + e].tau) == t) ++e;
+            if (t != kTauDummy) {
+                const int v[3] = {tau[t].pos / 49 - 3, (tau[t].pos / 7) % 7 - 3, tau[t].pos % 7 - 3};
+                int bytes = 8 * (e - r);
+                uint16_t sign[3] = {0, 0, 0};
+                for (int a = 0; a < 3; ++a)
+                    if (v[a] == 1 || v[a] == 2) sign[a] = static_cast<uint16_t>(bytes), bytes *= 2;
+                for (int q = r; q < e; ++q) {
+                    RowInfo& ri = rows[16 * b + q];
+                    ri.off = static_cast<uint32_t>(off + 8 * (q - r));
+                    for (int a = 0; a < 3; ++a) ri.sign[a] = sign[a];
+                }
+                off += bytes;
             }
-            if (t != kTauDummy) off += nvar[t] * (e - r);
             r = e;
         }
     }
@@ -918,8 +964,8 @@ int prepare_m2l_f64(Context* c) {
     HFMM_HIP(c, hipMemcpy(c->d_m2lrows.ptr, rows.data(), rbytes, hipMemcpyHostToDevice));
     TauInfo* dtau = reinterpret_cast<TauInfo*>(c->d_m2lrows.as<char>() + rbytes);
     HFMM_HIP(c, hipMemcpy(dtau, tau, sizeof(tau), hipMemcpyHostToDevice));
-    HFMM_TRY(ensure(c, c->d_m2ltab, tab.size()));
-    HFMM_HIP(c, hipMemcpy(c->d_m2ltab.ptr, tab.data(), tab.size(), hipMemcpyHostToDevice));
+    HFMM_TRY(ensure(c, c->d_m2ltab, sizeof(uint16_t) * slot_tau.size()));
+    HFMM_HIP(c, hipMemcpy(c->d_m2ltab.ptr, slot_tau.data(), sizeof(uint16_t) * slot_tau.size(), hipMemcpyHostToDevice));
 #define CALL(P) pack_impl<P>(c, nrb, dtau)
     HFMM_DISPATCH(c->order(), CALL)
 #undef CALL
