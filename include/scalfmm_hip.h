@@ -239,16 +239,16 @@ int hfmm_get_global_operators(hfmm_ctx* ctx, int32_t* rank, double* U, double* B
  * picks worse tile shapes.  No counterpart in the reference. */
 int hfmm_set_stream_overlap(hfmm_ctx* ctx, int32_t enable);
 
-/* Near field of the big leaves in the mixed forms (default on): each unordered
+/* Near field of the big leaves (default on): each unordered
  * pair of two neighbour leaves with more than 64 particles is evaluated once
  * and added to both particles, as the reference's P2POuter and its algorithms'
  * opposite-direction calls do (FChebSymKernel.hpp:468-478,
  * FGroupSeqAlgorithm.hpp:343-394, FP2P.hpp:103-171).  The source-side sums of
  * a pair go through per-(particle, neighbour work item) slots in device memory
  * that a second kernel adds in a fixed order, so results do not depend on the
- * launch.  Off: every ordered pair is evaluated by its target's kernel.  The
- * FP64 form always evaluates ordered pairs.  A tree whose slots would need
- * more than a quarter of the free device memory falls back to ordered pairs. */
+ * launch.  Off: every ordered pair is evaluated by its target's kernel.  A
+ * tree whose slots would need more than a quarter of the free device memory
+ * falls back to ordered pairs. */
 int hfmm_set_p2p_mutual(hfmm_ctx* ctx, int32_t enable);
 
 /* The state of the cells (multipoles and locals) between evaluations.

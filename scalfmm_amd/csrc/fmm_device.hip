@@ -441,6 +441,23 @@ __global__ __launch_bounds__(256) void k_l2p_lagrange(int64_t n, const int32_t* 
     }
 }
 
+// 1/sqrt(r2): v_rsq_f64 (about 26 bits) and one third-order step,
+// y (1 + e/2 + 3 e^2/8) with e = 1 - r2 y^2, whose error is of the order e^3:
+// 5 operations where two Newton steps take 7.
+__device__ __forceinline__ double rsqrt_f64(double r2) {
+    const double y = __builtin_amdgcn_rsq(r2);
+    const double e = fma(-(r2 * y), y, 1.);
+    return fma(y * e, fma(0.375, e, 0.5), y);
+}
+
+// The same for any r2: 1/0 = inf and 1/inf = 0, where the step would give NaN
+// (fmin drops the NaN of e).
+__device__ __forceinline__ double rsqrt_f64_any(double r2) {
+    const double y = __builtin_amdgcn_rsq(r2);
+    const double e = fmin(fma(-(r2 * y), y, 1.), 0.5);
+    return fma(y * e, fma(0.375, e, 0.5), y);
+}
+
 // ---------------------------------------------------------------------------
 // P2P: one thread per target particle, sources over its own leaf and the 26
 // neighbour slots; writes (initialises) the sorted results.
@@ -460,7 +477,7 @@ __global__ __launch_bounds__(256) void k_p2p_f64(int64_t n, const int32_t* __res
         for (int j = j0; j < j1; ++j) {
             if (j == i) continue;
             const double dx = tx - sp[j], dy = ty - sp[n + j], dz = tz - sp[2 * n + j];
-            const double inv = 1.0 / sqrt(dx * dx + dy * dy + dz * dz);
+            const double inv = rsqrt_f64_any(dx * dx + dy * dy + dz * dz);
             const double inv3 = inv * inv * inv;
             const double qs = sp[3 * n + j];
             pot += inv * qs;
@@ -499,7 +516,7 @@ __global__ __launch_bounds__(256) void k_p2p_f64_rhs(int64_t n, const int32_t* _
         for (int j = j0; j < j1; ++j) {
             if (j == i) continue;
             const double dx = tx - sp[j], dy = ty - sp[n + j], dz = tz - sp[2 * n + j];
-            const double inv = 1.0 / sqrt(dx * dx + dy * dy + dz * dz);
+            const double inv = rsqrt_f64_any(dx * dx + dy * dy + dz * dz);
             const double inv3 = inv * inv * inv;
             const double* q = qc + static_cast<int64_t>(j) * R;
 #pragma unroll
@@ -526,19 +543,11 @@ __global__ __launch_bounds__(256) void k_p2p_f64_rhs(int64_t n, const int32_t* _
 // items of kP2PItem consecutive targets of one leaf (two per lane) and walks
 // the 27 neighbour leaves in blocks of 8 sources.  Every source address is
 // wave-uniform, so the sources arrive through scalar loads into SGPRs and
-// feed the FP64 arithmetic as scalar operands (no LDS, no barriers).  1/r is
-// v_rsq_f64 refined by two Newton steps, y <- y (3 - r^2 y^2) / 2.  A block
+// feed the FP64 arithmetic as scalar operands (no LDS, no barriers).  A block
 // running past the leaf's end masks the extra sources (the sorted arrays are
 // padded, so the reads stay in bounds).  Sources are summed in the same order
 // as k_p2p_f64.
 constexpr int kP2PBlock64 = 8;
-
-__device__ __forceinline__ double rsqrt_f64(double r2) {
-    double y = __builtin_amdgcn_rsq(r2);
-    y = y * fma(-0.5 * r2, y * y, 1.5);
-    y = y * fma(-0.5 * r2, y * y, 1.5);
-    return y;
-}
 
 template <bool MASK>
 __device__ __forceinline__ void pair_f64(const double (&t)[3], double sx, double sy, double sz, double sq, bool skip,
@@ -554,9 +563,9 @@ __device__ __forceinline__ void pair_f64(const double (&t)[3], double sx, double
     acc[3] -= qi3 * dz;
 }
 
-template <bool SELF>
+template <bool SELF, int T>
 __device__ __forceinline__ void p2p_f64_leaf(const double* __restrict__ sp, int64_t n, int j0, int j1,
-                                             const double (&t)[2][3], const int (&ti)[2], double (&acc)[2][4]) {
+                                             const double (&t)[T][3], const int (&ti)[T], double (&acc)[T][4]) {
     int jb = j0;
     for (; jb + kP2PBlock64 <= j1; jb += kP2PBlock64) {
 #pragma unroll
@@ -564,7 +573,7 @@ __device__ __forceinline__ void p2p_f64_leaf(const double* __restrict__ sp, int6
             const int j = jb + jj;
             const double sx = sp[j], sy = sp[n + j], sz = sp[2 * n + j], sq = sp[3 * n + j];
 #pragma unroll
-            for (int u = 0; u < 2; ++u) pair_f64<SELF>(t[u], sx, sy, sz, sq, j == ti[u], acc[u]);
+            for (int u = 0; u < T; ++u) pair_f64<SELF>(t[u], sx, sy, sz, sq, j == ti[u], acc[u]);
         }
     }
     if (jb < j1) {
@@ -574,7 +583,7 @@ __device__ __forceinline__ void p2p_f64_leaf(const double* __restrict__ sp, int6
             const double sx = sp[j], sy = sp[n + j], sz = sp[2 * n + j], sq = sp[3 * n + j];
             const bool past = j >= j1;
 #pragma unroll
-            for (int u = 0; u < 2; ++u) pair_f64<true>(t[u], sx, sy, sz, sq, past || (SELF && j == ti[u]), acc[u]);
+            for (int u = 0; u < T; ++u) pair_f64<true>(t[u], sx, sy, sz, sq, past || (SELF && j == ti[u]), acc[u]);
         }
     }
 }
@@ -620,6 +629,202 @@ __global__ __launch_bounds__(256) void k_p2p_f64_big(const int2* __restrict__ it
             res[3 * n + ti[u]] = acc[u][3];
         }
     }
+}
+
+// Mutual FP64 P2P of the big leaves: each unordered pair of two big neighbour
+// leaves once, for both particles, in the scheme of the mixed form's kernel (p2p_mixed.hip): a work item is
+// up to 64 T targets of big leaf A, stationary in registers; its own leaf and
+// its small neighbours are evaluated pair by pair; each big forward neighbour B
+// (slots 0..12) is streamed in chunks of 64 sources, staged twice in a row in
+// the wave's LDS, so that at step k lane i reads source (i + k) mod 64.  The
+// source-side sum moves one lane down per step with its source, so that after
+// 64 steps lane i holds the sum of source (i + 63) mod 64 and writes it to B's
+// slot for this item; k_p2p_f64_combine adds a particle's slots in order: no
+// atomics, the same bits on every run.  FP64 needs no phases.
+// Issue slots of 4 cycles per unordered pair, T = 4: 3 differences, 3 for r^2,
+// 4 for v_rsq_f64, 5 refinement, 2 for 1/r^3, 2 charge products, 8 FMAs, 3 for
+// the rotation (8 DPP moves and 4 adds per source and step) = 30, against 2 x 22
+// for two ordered pairs: 21.5 ms for the 2.8e10 unordered pairs of 1.25M Plummer
+// particles at height 7, of which it takes 24.7 ms (the ordered kernel 56 ms).
+__device__ __forceinline__ double rol1_f64(double v) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const int lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(b), 0x134, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(b >> 32), 0x134, 0xF, 0xF, false);
+    return __builtin_bit_cast(double, (static_cast<uint64_t>(static_cast<uint32_t>(hi)) << 32) | static_cast<uint32_t>(lo));
+}
+
+template <int T>
+__device__ __forceinline__ void p2p_f64_mutual_item(const int32_t* __restrict__ lstart, const int32_t* __restrict__ slots,
+                                                    const double* __restrict__ sp, int64_t n,
+                                                    const int32_t* __restrict__ csoff,
+                                                    const int64_t* __restrict__ csbase, d4* __restrict__ cpart,
+                                                    double* __restrict__ res, double2* sxy, double2* szq, int leaf,
+                                                    int first, int tend, int tile, int part, int parts, int lane) {
+    int ti[T];
+    double t[T][3], qt[T], acc[T][4];
+#pragma unroll
+    for (int u = 0; u < T; ++u) {
+        ti[u] = first + 64 * u + lane;
+        const bool ok = ti[u] < tend;  // past the item: a copy of its first target with charge 0, never written
+        const int tt = ok ? ti[u] : first;
+        for (int d = 0; d < 3; ++d) t[u][d] = sp[d * n + tt];
+        qt[u] = ok ? sp[3 * n + tt] : 0.;
+        for (int k = 0; k < 4; ++k) acc[u][k] = 0.;
+    }
+    const int l0 = __builtin_amdgcn_readfirstlane(lstart[leaf]), l1 = __builtin_amdgcn_readfirstlane(lstart[leaf + 1]);
+    // the part's range of the chunks of 64 sources: the leaf's own, then those of
+    // its big forward neighbours
+    int nchunk = (l1 - l0 + 63) / 64;
+    for (int s = 0; s < kNbrForward; ++s) {
+        const int nb = __builtin_amdgcn_readfirstlane(slots[static_cast<int64_t>(leaf) * kNbrSlots + s]);
+        if (nb < 0) continue;
+        const int nbn = __builtin_amdgcn_readfirstlane(lstart[nb + 1] - lstart[nb]);
+        if (nbn > kP2PBig) nchunk += (nbn + 63) / 64;
+    }
+    int c0 = static_cast<int>(static_cast<int64_t>(part) * nchunk / parts);
+    int c1 = static_cast<int>(static_cast<int64_t>(part + 1) * nchunk / parts);
+    // ordered pairs: the leaf itself, and in part 0 its small neighbours
+    if (l0 + 64 * c0 < l1) p2p_f64_leaf<true, T>(sp, n, l0 + 64 * c0, min(l1, l0 + 64 * c1), t, ti, acc);
+    for (int s = 0; s < (part ? 0 : kNbrSlots); ++s) {
+        const int nb = __builtin_amdgcn_readfirstlane(slots[static_cast<int64_t>(leaf) * kNbrSlots + s]);
+        if (nb < 0) continue;
+        const int j0 = __builtin_amdgcn_readfirstlane(lstart[nb]);
+        const int j1 = __builtin_amdgcn_readfirstlane(lstart[nb + 1]);
+        if (j1 - j0 <= kP2PBig) p2p_f64_leaf<false, T>(sp, n, j0, j1, t, ti, acc);
+    }
+    c0 -= (l1 - l0 + 63) / 64;
+    c1 -= (l1 - l0 + 63) / 64;
+    // mutual pairs: the big forward neighbours
+    for (int s = 0; s < kNbrForward && c1 > 0; ++s) {
+        const int nb = __builtin_amdgcn_readfirstlane(slots[static_cast<int64_t>(leaf) * kNbrSlots + s]);
+        if (nb < 0) continue;
+        const int j0 = __builtin_amdgcn_readfirstlane(lstart[nb]);
+        const int j1 = __builtin_amdgcn_readfirstlane(lstart[nb + 1]);
+        const int nbn = j1 - j0;
+        if (nbn <= kP2PBig) continue;
+        const int jbeg = j0 + 64 * max(c0, 0), jend = min(j1, j0 + 64 * c1);
+        c0 -= (nbn + 63) / 64;
+        c1 -= (nbn + 63) / 64;
+        // this item's slot in B (A is B's backward neighbour in slot 25 - s)
+        const int slot = __builtin_amdgcn_readfirstlane(csoff[static_cast<int64_t>(nb) * kNbrForward + 12 - s]) + tile;
+        d4* cp = cpart + (csbase[nb] + static_cast<int64_t>(slot) * nbn);
+        for (int cb = jbeg; cb < jend; cb += 64) {
+            const int js = cb + lane;
+            const int jj = js < j1 ? js : j0;  // past the leaf: a charge-free copy of its first source
+            const double2 xy = make_double2(sp[jj], sp[n + jj]);
+            const double2 zq = make_double2(sp[2 * n + jj], js < j1 ? sp[3 * n + jj] : 0.);
+            sxy[lane] = sxy[lane + 64] = xy;
+            szq[lane] = szq[lane + 64] = zq;
+            // the wave's LDS accesses run in order; the fence keeps the compiler
+            // from moving other lanes' reads above these writes
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            double sa[4] = {0., 0., 0., 0.};
+#pragma unroll 8
+            for (int k = 0; k < 64; ++k) {
+                const double2 a = sxy[lane + k], b = szq[lane + k];
+                double cs[4];
+#pragma unroll
+                for (int u = 0; u < T; ++u) {
+                    const double dx = t[u][0] - a.x, dy = t[u][1] - a.y, dz = t[u][2] - b.x;
+                    const double inv = rsqrt_f64(fma(dz, dz, fma(dy, dy, dx * dx)));
+                    const double inv3 = inv * (inv * inv);
+                    const double a3 = b.y * inv3, b3 = qt[u] * inv3;
+                    acc[u][0] = fma(b.y, inv, acc[u][0]);
+                    acc[u][1] = fma(-a3, dx, acc[u][1]);
+                    acc[u][2] = fma(-a3, dy, acc[u][2]);
+                    acc[u][3] = fma(-a3, dz, acc[u][3]);
+                    cs[0] = u ? fma(qt[u], inv, cs[0]) : qt[u] * inv;
+                    cs[1] = u ? fma(b3, dx, cs[1]) : b3 * dx;
+                    cs[2] = u ? fma(b3, dy, cs[2]) : b3 * dy;
+                    cs[3] = u ? fma(b3, dz, cs[3]) : b3 * dz;
+                }
+#pragma unroll
+                for (int q = 0; q < 4; ++q) sa[q] = rol1_f64(sa[q]) + cs[q];
+            }
+            const int jo = cb + ((lane + 63) & 63);
+            if (jo < j1) cp[jo - j0] = d4{sa[0], sa[1], sa[2], sa[3]};
+            // the next chunk rewrites the sources only after these reads
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        }
+    }
+    // part 0 starts the results, the others fill the leaf's last slots
+    d4* own = cpart + (csbase[leaf + 1] - static_cast<int64_t>(parts - part) * (l1 - l0) - l0);
+#pragma unroll
+    for (int u = 0; u < T; ++u) {
+        if (ti[u] >= tend) continue;
+        if (part) {
+            own[ti[u]] = d4{acc[u][0], acc[u][1], acc[u][2], acc[u][3]};
+            continue;
+        }
+        res[ti[u]] = acc[u][0];
+        res[n + ti[u]] = acc[u][1];
+        res[2 * n + ti[u]] = acc[u][2];
+        res[3 * n + ti[u]] = acc[u][3];
+    }
+}
+
+__global__ __launch_bounds__(256) void k_p2p_f64_mutual(const int2* __restrict__ items, const int32_t* __restrict__ nitems,
+                                                       const int32_t* __restrict__ lstart,
+                                                       const int32_t* __restrict__ slots, const double* __restrict__ sp,
+                                                       int64_t n, const int32_t* __restrict__ csoff,
+                                                       const int64_t* __restrict__ csbase,
+                                                       const int32_t* __restrict__ csparts, d4* __restrict__ cpart,
+                                                       int32_t* __restrict__ next, double* __restrict__ res) {
+    static_assert(kP2PMutualItem == 256, "work item = one wave x up to 4 targets");
+    __shared__ double2 s_xy[4][128], s_zq[4][128];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int total = *nitems;
+    // parts of work items claimed one at a time, costliest items first (kP2PMaxParts
+    // claims each, most items have one part); every wave leaves once the counter
+    // passes the last
+    for (;;) {
+        int claim = 0;
+        if (lane == 0) claim = atomicAdd(next, 1);
+        const int at = __builtin_amdgcn_readfirstlane(__shfl(claim, 0));
+        const int it = at / kP2PMaxParts, part = at % kP2PMaxParts;
+        if (it >= total) break;
+        const int2 item = items[it];
+        const int leaf = __builtin_amdgcn_readfirstlane(item.x);
+        const int first = __builtin_amdgcn_readfirstlane(item.y);
+        const int parts = __builtin_amdgcn_readfirstlane(csparts[leaf]);
+        if (part >= parts) continue;
+        const int l0 = __builtin_amdgcn_readfirstlane(lstart[leaf]);
+        const int tend = min(__builtin_amdgcn_readfirstlane(lstart[leaf + 1]), first + kP2PMutualItem);
+        const int tile = (first - l0) / kP2PMutualItem;
+        // as many targets per lane as the item needs: the last item of a leaf
+        // may hold a few
+#define ITEM(T) \
+    p2p_f64_mutual_item<T>(lstart, slots, sp, n, csoff, csbase, cpart, res, s_xy[wave], s_zq[wave], leaf, first, tend, tile, part, \
+                           parts, lane)
+        switch ((tend - first + 63) / 64) {
+            case 1: ITEM(1); break;
+            case 2: ITEM(2); break;
+            case 3: ITEM(3); break;
+            default: ITEM(4); break;
+        }
+#undef ITEM
+    }
+}
+
+// Adds the source-side sums of the mutual P2P to the big leaves' particles: one
+// thread per particle, its slots in order.
+__global__ __launch_bounds__(256) void k_p2p_f64_combine(int64_t n, const int32_t* __restrict__ pleaf,
+                                                        const int32_t* __restrict__ lstart,
+                                                        const int64_t* __restrict__ csbase,
+                                                        const d4* __restrict__ cpart, double* __restrict__ res) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int li = pleaf[i];
+    const int j0 = lstart[li], m = lstart[li + 1] - j0;
+    if (m <= kP2PBig) return;
+    const int64_t b0 = csbase[li];
+    const int64_t ns = (csbase[li + 1] - b0) / m;
+    if (ns == 0) return;
+    const d4* p = cpart + b0 + (i - j0);
+    d4 s = {0., 0., 0., 0.};
+    for (int64_t k = 0; k < ns; ++k) s += p[k * m];
+    for (int q = 0; q < 4; ++q) res[q * n + i] += s[q];
 }
 
 __global__ void k_mfma_probe(double* out) {
@@ -815,6 +1020,35 @@ int run_p2p(Context* c) {
                            sorted_results(c));
         prof_end(c);
         HFMM_TRY(check_launch(c, "p2p"));
+    }
+    if (c->p2p_items_cap == 0) return HFMM_OK;
+    if (c->p2p_mutual && c->p2p_mutual_on) {
+        // persistent grid: as many workgroups as fit on the device at once
+        static int resident[64] = {0};
+        if (c->device < 0 || c->device >= 64) return fail(c, HFMM_ERR_ARG, "device ordinal above 63");
+        if (resident[c->device] == 0) {
+            int per_cu = 0, cus = 0;
+            HFMM_HIP(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                            &per_cu, reinterpret_cast<const void*>(&k_p2p_f64_mutual), 256, 0));
+            HFMM_HIP(c, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device));
+            resident[c->device] = std::max(1, per_cu) * std::max(1, cus);
+        }
+        const int64_t want = (c->p2p_items_m_cap * kP2PMaxParts + 3) / 4;
+        const unsigned grid = static_cast<unsigned>(std::max<int64_t>(1, std::min<int64_t>(want, resident[c->device])));
+        HFMM_TRY(zero_device(c, p2p_mutual_next(c), sizeof(int32_t)));  // a fill kernel: capturable
+        prof_begin(c, "p2p_big");
+        hipLaunchKernelGGL(k_p2p_f64_mutual, dim3(grid), dim3(256), 0, c->stream, c->d_p2pitems_m.as<int2>(),
+                           p2p_mutual_item_count(c), c->d_leafstart.as<int32_t>(), c->d_p2p.as<int32_t>(),
+                           c->d_sorted.as<double>(), c->n, c->d_csoff.as<int32_t>(), c->d_csbase.as<int64_t>(),
+                           c->d_csparts.as<int32_t>(), c->d_cpart.as<d4>(), p2p_mutual_next(c), sorted_results(c));
+        prof_end(c);
+        HFMM_TRY(check_launch(c, "p2p_big"));
+        prof_begin(c, "p2p_combine");
+        hipLaunchKernelGGL(k_p2p_f64_combine, dim3(blocks256(c->n)), dim3(256), 0, c->stream, c->n,
+                           c->d_pleaf.as<int32_t>(), c->d_leafstart.as<int32_t>(), c->d_csbase.as<int64_t>(),
+                           c->d_cpart.as<d4>(), sorted_results(c));
+        prof_end(c);
+        return check_launch(c, "p2p_combine");
     }
     prof_begin(c, "p2p_big");
     hipLaunchKernelGGL(k_p2p_f64_big, dim3((p2p_tiled_grid(c) + 3) / 4), dim3(256), 0, c->stream,

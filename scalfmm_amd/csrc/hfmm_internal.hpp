@@ -21,6 +21,7 @@ constexpr int kTileTargets = 16;  // targets per M2L tile (the MFMA N dimension)
 constexpr int kP2PBig = 64;    // leaves with more particles run P2P through LDS-staged sources
 constexpr int kP2PItem = 128;  // targets per P2P work item of a big leaf (two per lane of a wave)
 constexpr int kP2PMutualItem = 256;  // targets per work item of the mutual mixed P2P (four per lane)
+constexpr int kP2PMaxParts = 32;  // parts of a work item of the mutual FP64 P2P
 constexpr int kNbrForward = 13;  // neighbour slots 0..12 (positions 0..12): the mutual P2P's forward half
 constexpr int kSortedPad = 16; // padding doubles after the sorted particle SoA
 constexpr int kWaveM2LMaxOrder = 6;  // highest order of the wave-level mixed M2L kernel
@@ -142,21 +143,23 @@ struct Context {
     DevBuf d_leafstart;                       // int32 [nleaf+1]
     DevBuf d_p2p;                             // int32 [nleaf][26]
     DevBuf d_p2pitems;                        // int2 (leaf, first target) work items of the big leaves
-    int64_t p2p_items_cap = 0;                // upper bound of the item count (the count itself is on the device)
-    // Mutual mixed P2P (each unordered pair of big leaves evaluated once): work
+    int64_t p2p_items_cap = 0;                // their number (0: no big leaf)
+    // Mutual P2P (each unordered pair of big leaves evaluated once): work
     // items of kP2PMutualItem targets, and the source-side sums that a leaf
     // receives from the items of its big backward neighbours (slots 13..25):
-    // per leaf 13 slot offsets (-1: none) and the first float4 of its slots
-    // (each slot holds one float4 per particle of the leaf)
+    // per leaf 13 slot offsets (-1: none) and the first entry of its slots
+    // (each slot holds one entry, potential and field, per particle of the leaf;
+    // four floats in the mixed forms, four doubles in FP64)
     bool p2p_mutual = false;                  // tables built and the partial buffer allocated
     bool p2p_mutual_on = true;                // hfmm_set_p2p_mutual (the ordered-pair kernel when off)
     DevBuf d_p2pitems_m;                      // int2 (leaf, first target), costliest first
     DevBuf d_itemkeys, d_itemidx, d_items_tmp; // sorting scratch of the mutual work items
     int64_t p2p_items_m_cap = 0;
     DevBuf d_csoff;                           // int32 [nleaf][13]
+    DevBuf d_csparts;                         // int32 [nleaf] parts of an item (FP64)
     DevBuf d_csbase;                          // int64 [nleaf + 1]
-    DevBuf d_cpart;                           // float4 source-side partial sums
-    int64_t cpart_units = 0;                  // float4 entries in use
+    DevBuf d_cpart;                           // source-side partial sums
+    int64_t cpart_units = 0;                  // entries in use
     DevBuf d_m2l;                             // int32 [cells of levels 2..h-1][189]
     int64_t m2l_off[kMaxLevels] = {0};        // offset (in cells) of a level in d_m2l
     DevBuf d_order;                           // int32 parity-sorted cell index per level (same offsets as d_m2l)
@@ -276,7 +279,7 @@ inline int64_t* p2p_mutual_units(Context* c) { return c->d_count.as<int64_t>() +
 // time; cleared before each launch).
 inline int32_t* p2p_mutual_next(Context* c) { return reinterpret_cast<int32_t*>(c->d_count.as<int64_t>() + 18); }
 // Builds the mutual P2P's work items and slot tables on a built tree and sizes
-// the partial buffer (mixed forms); leaves c->p2p_mutual false when the
+// the partial buffer; leaves c->p2p_mutual false when the
 // partial sums would exceed a quarter of the free device memory.
 int build_p2p_mutual_tables(Context* c);
 

@@ -529,6 +529,7 @@ int run_p2p_mixed(Context* c) {
         prof_end(c);
         HFMM_TRY(check_launch(c, "p2p_mixed"));
     }
+    if (c->p2p_items_cap == 0) return HFMM_OK;  // no big leaf
     if (!(c->p2p_mutual && c->p2p_mutual_on)) {
         const unsigned grid = (p2p_tiled_grid(c) + 3) / 4;
         prof_begin(c, "p2p_mixed_big");

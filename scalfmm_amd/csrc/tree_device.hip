@@ -560,10 +560,19 @@ int sort_p2p_items(Context* c, int2* items, const int32_t* nitems, int64_t cap) 
 // of neighbour B go to B's slot csoff[B][12 - s] + t, A being B's backward
 // neighbour in slot 25 - s.  Per big leaf B: the 13 offsets (one per backward
 // slot 13..25, -1 when that neighbour is absent or small) and units[B] =
-// (number of slots) x (particles of B) float4 entries.
+// (number of slots) x (particles of B) entries.
+// An item of the FP64 kernel is taken in parts[A] parts of about kP2PPartPairs
+// pairs, each a range of the sources of A itself and of its big forward
+// neighbours: one wave would need 14 ms for a central item of a Plummer set of
+// 120,000 particles at height 6 (256 targets, 70,000 sources).  Part 0 writes
+// the targets' results, each further part a slot of A's own, after those of the
+// backward neighbours.
+constexpr int64_t kP2PPartPairs = int64_t(1) << 18;
+
 __global__ __launch_bounds__(kBlock) void k_colslot_counts(int nleaf, const int32_t* __restrict__ lstart,
-                                                          const int32_t* __restrict__ slots,
-                                                          int32_t* __restrict__ csoff, int64_t* __restrict__ units) {
+                                                           const int32_t* __restrict__ slots, int split,
+                                                           int32_t* __restrict__ csoff, int64_t* __restrict__ units,
+                                                           int32_t* __restrict__ parts) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nleaf) return;
     const int m = lstart[i + 1] - lstart[i];
@@ -580,7 +589,18 @@ __global__ __launch_bounds__(kBlock) void k_colslot_counts(int nleaf, const int3
         }
         csoff[static_cast<int64_t>(i) * kNbrForward + b] = o;
     }
-    units[i] = static_cast<int64_t>(run) * m;
+    int k = 1;
+    if (split && m > kP2PBig) {
+        int64_t src = m;
+        for (int b = 0; b < kNbrForward; ++b) {
+            const int a = slots[static_cast<int64_t>(i) * kNbrSlots + b];
+            const int na = a < 0 ? 0 : lstart[a + 1] - lstart[a];
+            if (na > kP2PBig) src += na;
+        }
+        k = static_cast<int>(min(static_cast<int64_t>(kP2PMaxParts), 1 + src * min(m, kP2PMutualItem) / kP2PPartPairs));
+    }
+    parts[i] = k;
+    units[i] = static_cast<int64_t>(run + k - 1) * m;
 }
 
 int make_groups(Context* c, const uint64_t* keys, int64_t n, int shift, uint64_t* gkey, int32_t* gstart,
@@ -774,9 +794,7 @@ int build_tree_device(Context* c) {
     prof_end(c);
     HFMM_TRY(check_launch(c, "p2p_lists"));
     {
-        // items of the big leaves; their count stays on the device (slot 12 of d_count)
-        c->p2p_items_cap = n / kP2PItem + n / (kP2PBig + 1) + 1;
-        HFMM_TRY(ensure(c, c->d_p2pitems, sizeof(int2) * static_cast<size_t>(c->p2p_items_cap)));
+        // items of the big leaves (slot 12 of d_count: their number)
         HFMM_TRY(ensure(c, c->d_flags, sizeof(int32_t) * static_cast<size_t>(nl + 1)));
         HFMM_TRY(ensure(c, c->d_scan, sizeof(int32_t) * static_cast<size_t>(nl + 1)));
         prof_begin(c, "p2p_items");
@@ -786,6 +804,13 @@ int build_tree_device(Context* c) {
         HFMM_TRY(check_launch(c, "p2p_items"));
         HFMM_TRY(exclusive_scan<int32_t>(c, c->d_flags.as<int32_t>(), c->d_scan.as<int32_t>(), nl, p2p_item_count(c),
                                          "p2p_items"));
+        int32_t items = 0;
+        HFMM_HIP(c, hipMemcpyAsync(&items, p2p_item_count(c), sizeof(int32_t), hipMemcpyDeviceToHost, c->stream));
+        HFMM_HIP(c, hipStreamSynchronize(c->stream));
+        c->p2p_items_cap = items;
+    }
+    if (c->p2p_items_cap > 0) {
+        HFMM_TRY(ensure(c, c->d_p2pitems, sizeof(int2) * static_cast<size_t>(c->p2p_items_cap)));
         prof_begin(c, "p2p_items");
         hipLaunchKernelGGL(k_p2p_items<kP2PItem>, dim3(blocks_for(nl)), dim3(kBlock), 0, c->stream, static_cast<int>(nl),
                            c->d_leafstart.as<int32_t>(), c->d_scan.as<int32_t>(), c->d_p2pitems.as<int2>());
@@ -824,7 +849,7 @@ int build_tree_device(Context* c) {
     c->tree_built = true;
     c->evaluated = false;
     c->p2p_mutual = false;
-    if (is_mixed(c)) HFMM_TRY(build_p2p_mutual_tables(c));
+    if (c->p2p_items_cap > 0) HFMM_TRY(build_p2p_mutual_tables(c));
     return HFMM_OK;
 }
 
@@ -852,10 +877,11 @@ int build_p2p_mutual_tables(Context* c) {
                                                     c->p2p_items_m_cap)));
     HFMM_TRY(ensure(c, c->d_csoff, sizeof(int32_t) * static_cast<size_t>(nl) * kNbrForward));
     HFMM_TRY(ensure(c, c->d_csbase, sizeof(int64_t) * static_cast<size_t>(nl + 1)));
+    HFMM_TRY(ensure(c, c->d_csparts, sizeof(int32_t) * static_cast<size_t>(nl)));
     int64_t* base = c->d_csbase.as<int64_t>();
     prof_begin(c, "p2p_items");
     hipLaunchKernelGGL(k_colslot_counts, dim3(blocks_for(nl)), dim3(kBlock), 0, c->stream, static_cast<int>(nl), lstart,
-                       c->d_p2p.as<int32_t>(), c->d_csoff.as<int32_t>(), base);
+                       c->d_p2p.as<int32_t>(), is_mixed(c) ? 0 : 1, c->d_csoff.as<int32_t>(), base, c->d_csparts.as<int32_t>());
     prof_end(c);
     HFMM_TRY(check_launch(c, "p2p_items"));
     HFMM_TRY(exclusive_scan<int64_t>(c, base, base, nl, p2p_mutual_units(c), "p2p_items"));
@@ -864,7 +890,7 @@ int build_p2p_mutual_tables(Context* c) {
     HFMM_HIP(c, hipStreamSynchronize(c->stream));
     // base[nl] = the total, so a leaf's slot count is (base[i+1] - base[i]) / n_i
     HFMM_HIP(c, hipMemcpyAsync(base + nl, p2p_mutual_units(c), sizeof(int64_t), hipMemcpyDeviceToDevice, c->stream));
-    const size_t bytes = sizeof(float) * 4 * static_cast<size_t>(units > 0 ? units : 1);
+    const size_t bytes = (is_mixed(c) ? sizeof(float) : sizeof(double)) * 4 * static_cast<size_t>(units > 0 ? units : 1);
     if (bytes > c->d_cpart.bytes) {
         size_t free_b = 0, total_b = 0;
         HFMM_HIP(c, hipMemGetInfo(&free_b, &total_b));

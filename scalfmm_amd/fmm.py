@@ -192,7 +192,7 @@ class Engine:
         self._check(self._L.hfmm_set_stream_overlap(self.h, 1 if on else 0))
 
     def set_p2p_mutual(self, on=True):
-        """Mixed forms: each unordered pair of two big neighbour leaves once (default on)."""
+        """Each unordered pair of two big neighbour leaves once (default on)."""
         self._check(self._L.hfmm_set_p2p_mutual(self.h, 1 if on else 0))
 
     def reset_cells(self):
