@@ -4,9 +4,11 @@
 // (Tests/Kernels/DirectAlgorithm.cpp:203-215, Src/Kernels/P2P/FP2P.hpp:80-101).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <mutex>
 #include <string>
 
+#include "fmm_common.hpp"
 #include "hfmm_internal.hpp"
 
 namespace hfmm {
@@ -15,17 +17,21 @@ namespace {
 constexpr int kDirectBlock = 256;
 constexpr int kDirectTargets = 8;  // targets per workgroup (sources are read once for all of them)
 
-// A workgroup per kDirectTargets targets: the threads stride over all
-// sources, then a tree reduction in LDS per target.  Force convention
-// F = q_t * sum_j -q_j d / r^3, the FMM's.
+// A workgroup per kDirectTargets targets and share of the sources: the threads
+// stride over the share, then a tree reduction in LDS per target.  Force
+// convention F = q_t * sum_j -q_j d / r^3, the FMM's.  With several shares the
+// sums go to part[share][4][nt] and k_direct_sum adds them in order.  One
+// share per target group left 3,001 targets to 376 workgroups (1.4 per CU) and
+// one target to a single one.
 __global__ __launch_bounds__(kDirectBlock) void k_direct(int64_t n, const double* __restrict__ x,
                                                         const double* __restrict__ y, const double* __restrict__ z,
                                                         const double* __restrict__ q,
                                                         const int64_t* __restrict__ targets, int64_t nt,
-                                                        double* __restrict__ out) {
+                                                        double* __restrict__ out, double* __restrict__ part) {
     __shared__ double red[4][kDirectBlock];
     int64_t t[kDirectTargets];
     double tx[kDirectTargets], ty[kDirectTargets], tz[kDirectTargets], acc[kDirectTargets][4];
+#pragma unroll
     for (int u = 0; u < kDirectTargets; ++u) {
         const int64_t g = static_cast<int64_t>(blockIdx.x) * kDirectTargets + u;
         t[u] = g < nt ? targets[g] : -1;
@@ -35,13 +41,16 @@ __global__ __launch_bounds__(kDirectBlock) void k_direct(int64_t n, const double
         tz[u] = z[tt];
         for (int k = 0; k < 4; ++k) acc[u][k] = 0.;
     }
-    for (int64_t j = threadIdx.x; j < n; j += kDirectBlock) {
+    const int64_t j0 = n * blockIdx.y / gridDim.y, j1 = n * (blockIdx.y + 1) / gridDim.y;
+    for (int64_t j = j0 + threadIdx.x; j < j1; j += kDirectBlock) {
         const double xj = x[j], yj = y[j], zj = z[j], qj = q[j];
+#pragma unroll
         for (int u = 0; u < kDirectTargets; ++u) {
-            if (j == t[u]) continue;
             const double dx = tx[u] - xj, dy = ty[u] - yj, dz = tz[u] - zj;
-            const double inv = 1.0 / sqrt(dx * dx + dy * dy + dz * dz);
-            const double qi = qj * inv;
+            double inv = rsqrt_f64_any(dx * dx + dy * dy + dz * dz);
+            const double q1 = j == t[u] ? 0. : qj;
+            inv = j == t[u] ? 0. : inv;
+            const double qi = q1 * inv;
             const double qi3 = qi * inv * inv;
             acc[u][0] += qi;
             acc[u][1] -= qi3 * dx;
@@ -59,14 +68,31 @@ __global__ __launch_bounds__(kDirectBlock) void k_direct(int64_t n, const double
         }
         if (threadIdx.x == 0 && t[u] >= 0) {
             const int64_t g = static_cast<int64_t>(blockIdx.x) * kDirectTargets + u;
-            const double qt = q[t[u]];
-            out[g] = red[0][0];
-            out[nt + g] = red[1][0] * qt;
-            out[2 * nt + g] = red[2][0] * qt;
-            out[3 * nt + g] = red[3][0] * qt;
+            if (gridDim.y > 1) {
+                for (int k = 0; k < 4; ++k) part[(blockIdx.y * 4 + k) * nt + g] = red[k][0];
+            } else {
+                const double qt = q[t[u]];
+                out[g] = red[0][0];
+                out[nt + g] = red[1][0] * qt;
+                out[2 * nt + g] = red[2][0] * qt;
+                out[3 * nt + g] = red[3][0] * qt;
+            }
         }
         __syncthreads();
     }
+}
+
+__global__ __launch_bounds__(kDirectBlock) void k_direct_sum(const double* __restrict__ q,
+                                                            const int64_t* __restrict__ targets, int64_t nt, int shares,
+                                                            const double* __restrict__ part, double* __restrict__ out) {
+    const int64_t g = static_cast<int64_t>(blockIdx.x) * kDirectBlock + threadIdx.x;
+    if (g >= nt) return;
+    double s[4] = {0., 0., 0., 0.};
+    for (int i = 0; i < shares; ++i)
+        for (int k = 0; k < 4; ++k) s[k] += part[(static_cast<int64_t>(i) * 4 + k) * nt + g];
+    const double qt = q[targets[g]];
+    out[g] = s[0];
+    for (int k = 1; k < 4; ++k) out[k * nt + g] = s[k] * qt;
 }
 
 // Staging of hfmm_direct_noalloc: the target indices (kDirectStaticTargets
@@ -81,13 +107,34 @@ constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 void* g_scratch_ptr[kMaxDevices] = {};  // device address of `scratch` per device
 
+// Shares of the sources: enough for kDirectBlocks workgroups, a round of the
+// threads or more each, partial sums (32 bytes per target and share) within the
+// static staging beside the 40 bytes per target, so that both entry points
+// split, and sum, alike.
+constexpr int64_t kDirectBlocks = 2048;
+
+int direct_shares(int64_t n, int64_t nt) {
+    const int64_t blocks = (nt + kDirectTargets - 1) / kDirectTargets;
+    int64_t s = (kDirectBlocks + blocks - 1) / blocks;
+    s = std::min(s, (n + kDirectBlock - 1) / kDirectBlock);
+    s = std::min<int64_t>(s, (kDirectStaticTargets * 40 - nt * 40) / (nt * 32));
+    return static_cast<int>(std::max<int64_t>(1, s));
+}
+
 // Launch of k_direct over c's particles for nt targets whose indices are at
-// device address dt, results (four arrays of nt) at dout.
+// device address dt, results (four arrays of nt) at dout, followed by room for
+// the partial sums of direct_shares.
 int launch_direct(Context* c, int64_t nt, const int64_t* dt, double* dout) {
     const int64_t blocks = (nt + kDirectTargets - 1) / kDirectTargets;
-    hipLaunchKernelGGL(k_direct, dim3(static_cast<unsigned>(blocks)), dim3(kDirectBlock), 0, c->stream, c->n, c->x,
-                       c->y, c->z, c->q, dt, nt, dout);
-    return check_launch(c, "direct");
+    const int shares = direct_shares(c->n, nt);
+    double* part = dout + 4 * nt;
+    hipLaunchKernelGGL(k_direct, dim3(static_cast<unsigned>(blocks), static_cast<unsigned>(shares)), dim3(kDirectBlock), 0,
+                       c->stream, c->n, c->x, c->y, c->z, c->q, dt, nt, dout, part);
+    HFMM_TRY(check_launch(c, "direct"));
+    if (shares == 1) return HFMM_OK;
+    hipLaunchKernelGGL(k_direct_sum, dim3(static_cast<unsigned>((nt + kDirectBlock - 1) / kDirectBlock)),
+                       dim3(kDirectBlock), 0, c->stream, c->q, dt, nt, shares, part, dout);
+    return check_launch(c, "direct_sum");
 }
 
 // Copies the four result arrays at dout (nt each) into the caller's host
@@ -130,7 +177,7 @@ int direct_sum_noalloc(Context* c, int64_t nt, const int64_t* targets, double* p
     }
     if (!base) return fail(c, HFMM_ERR_STATE, "direct_noalloc: the static staging of this device is not set up");
     int64_t* dt = static_cast<int64_t*>(base);
-    double* dout = reinterpret_cast<double*>(dt + kDirectStaticTargets);
+    double* dout = reinterpret_cast<double*>(dt + nt);
     // every call rewrites the staging it reads: the target indices here, each
     // result entry by the kernel (one per target), so nothing needs clearing
     if (hipMemcpyAsync(dt, targets, sizeof(int64_t) * nt, hipMemcpyHostToDevice, c->stream) != hipSuccess)
@@ -140,17 +187,14 @@ int direct_sum_noalloc(Context* c, int64_t nt, const int64_t* targets, double* p
 }
 
 int direct_sum(Context* c, int64_t nt, const int64_t* targets, double* pot, double* fx, double* fy, double* fz) {
-    DevBuf dt, dout;
-    int st = ensure(c, dt, sizeof(int64_t) * nt);
-    if (st == HFMM_OK) st = ensure(c, dout, sizeof(double) * 4 * nt);
-    if (st == HFMM_OK && hipMemcpyAsync(dt.ptr, targets, sizeof(int64_t) * nt, hipMemcpyHostToDevice, c->stream) !=
-                             hipSuccess)
-        st = fail(c, HFMM_ERR_DEVICE, "direct: target copy failed");
-    if (st == HFMM_OK) st = launch_direct(c, nt, dt.as<int64_t>(), dout.as<double>());
-    if (st == HFMM_OK) st = copy_direct_results(c, nt, dout.as<double>(), pot, fx, fy, fz);
-    release(dt);
-    release(dout);
-    return st;
+    // staging kept by the context: indices, results, partial sums
+    HFMM_TRY(ensure(c, c->d_direct, static_cast<size_t>(nt) * (40 + 32 * direct_shares(c->n, nt))));
+    int64_t* dt = c->d_direct.as<int64_t>();
+    double* dout = reinterpret_cast<double*>(dt + nt);
+    if (hipMemcpyAsync(dt, targets, sizeof(int64_t) * nt, hipMemcpyHostToDevice, c->stream) != hipSuccess)
+        return fail(c, HFMM_ERR_DEVICE, "direct: target copy failed");
+    HFMM_TRY(launch_direct(c, nt, dt, dout));
+    return copy_direct_results(c, nt, dout, pot, fx, fy, fz);
 }
 
 }  // namespace hfmm

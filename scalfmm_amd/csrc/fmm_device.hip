@@ -441,23 +441,6 @@ __global__ __launch_bounds__(256) void k_l2p_lagrange(int64_t n, const int32_t* 
     }
 }
 
-// 1/sqrt(r2): v_rsq_f64 (about 26 bits) and one third-order step,
-// y (1 + e/2 + 3 e^2/8) with e = 1 - r2 y^2, whose error is of the order e^3:
-// 5 operations where two Newton steps take 7.
-__device__ __forceinline__ double rsqrt_f64(double r2) {
-    const double y = __builtin_amdgcn_rsq(r2);
-    const double e = fma(-(r2 * y), y, 1.);
-    return fma(y * e, fma(0.375, e, 0.5), y);
-}
-
-// The same for any r2: 1/0 = inf and 1/inf = 0, where the step would give NaN
-// (fmin drops the NaN of e).
-__device__ __forceinline__ double rsqrt_f64_any(double r2) {
-    const double y = __builtin_amdgcn_rsq(r2);
-    const double e = fmin(fma(-(r2 * y), y, 1.), 0.5);
-    return fma(y * e, fma(0.375, e, 0.5), y);
-}
-
 // ---------------------------------------------------------------------------
 // P2P: one thread per target particle, sources over its own leaf and the 26
 // neighbour slots; writes (initialises) the sorted results.

@@ -158,6 +158,7 @@ struct Context {
     DevBuf d_csoff;                           // int32 [nleaf][13]
     DevBuf d_csparts;                         // int32 [nleaf] parts of an item (FP64)
     DevBuf d_csbase;                          // int64 [nleaf + 1]
+    DevBuf d_direct;                          // staging of hfmm_direct
     DevBuf d_cpart;                           // source-side partial sums
     int64_t cpart_units = 0;                  // entries in use
     DevBuf d_m2l;                             // int32 [cells of levels 2..h-1][189]
