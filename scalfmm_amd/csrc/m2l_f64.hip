@@ -581,9 +581,12 @@ __device__ __forceinline__ void down_body(const M2LArgs& a, const SmemLayout& sl
                 bv[r][c][0] = x[0];
                 bv[r][c][1] = x[1];
             }
-        auto products = [&](int s) {  // K step s of the row blocks
+        // quarter q of the step's K steps, row block by row block: both tile shapes
+        // add a target's terms in the same order (equal bits whatever the shape)
+        auto products = [&](int q) {
 #pragma unroll
-            for (int r = 0; r < RB; ++r)
+            for (int k = RB * q; k < RB * (q + 1); ++k) {
+                const int r = k / 4, s = k % 4;
 #pragma unroll
                 for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -591,6 +594,7 @@ __device__ __forceinline__ void down_body(const M2LArgs& a, const SmemLayout& sl
                         acc[t][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(
                             s & 1 ? av[r][t][s / 2].y : av[r][t][s / 2].x,
                             s & 1 ? bv[r][c][s / 2].y : bv[r][c][s / 2].x, acc[t][c], 0, 0, 0);
+            }
         };
         operators(s_list[i + 1 < nact ? i + 1 : i], nv);
         M2L_FENCE;

@@ -41,3 +41,26 @@ def test_m2l_tiles(dist, n, h, p):
     for got, want in zip(e.results(), ref[:4]):
         assert rel(got, want) < 1e-12
     e.close()
+
+
+def test_m2l_tile_shapes_agree():
+    """A set alone (one column tile per workgroup) and among others (two): the
+    same bits, since a target's terms are added in the same order."""
+    x, y, z, q = uniform_cube(36003, 23)
+    for p in (5, 7):
+        e = Engine(6, 1.0, CENTER, p)
+        off = [0, 12001, 24002, 36003]
+        e.set_particle_sets(off, x, y, z, q)
+        e.build_tree()
+        e.evaluate()
+        got = e.results()
+        e.close()
+        e = Engine(6, 1.0, CENTER, p)
+        for a, b in zip(off, off[1:]):
+            e.set_particles(x[a:b], y[a:b], z[a:b], q[a:b])
+            e.build_tree()
+            assert sum(e.tree_info().n_cells) < 16384  # the other tile shape
+            e.evaluate()
+            for g, r in zip(got, e.results()):
+                assert np.array_equal(g[a:b], r)
+        e.close()
