@@ -577,6 +577,7 @@ int run_global_m2l(Context* c) {
     const int NR = (k + 15) / 16;
     if (NR <= kGlobalMfmaMaxTiles) {
         HFMM_TRY(prepare_global_mfma(c, 16 * NR));
+        HFMM_TRY(ensure_parity_order(c));
         int tiles = 0;
         const M2LLevels lv = make_levels(c, 16, tiles);
         if (tiles == 0) return HFMM_OK;

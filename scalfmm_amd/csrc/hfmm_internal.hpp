@@ -124,7 +124,7 @@ struct Context {
     // ---- tree
     bool tree_built = false;
     bool evaluated = false;
-    DevBuf d_keys, d_keys2, d_vals, d_vals2;  // sort buffers (uint64 / int32)
+    DevBuf d_keys, d_keys2, d_vals2;  // sort buffers (uint64 / int32)
     DevBuf d_hist;                            // radix histogram / scan scratch
     DevBuf d_scan_part;                       // scan partials
     DevBuf d_flags, d_scan;                   // int32 per element
@@ -137,13 +137,12 @@ struct Context {
     int64_t lvl_off[kMaxLevels + 1] = {0};    // offsets in the cell arrays
     int64_t total_cells = 0;
     DevBuf d_cellkey;                         // uint64 [total_cells]
-    DevBuf d_cellkey_tmp;                     // scratch per level
     DevBuf d_childstart;                      // int32 [total_cells + levels] (ncell[l]+1 per level)
     int64_t cs_off[kMaxLevels] = {0};
     DevBuf d_leafstart;                       // int32 [nleaf+1]
     DevBuf d_p2p;                             // int32 [nleaf][26]
     DevBuf d_p2pitems;                        // int2 (leaf, first target) work items of the big leaves
-    int64_t p2p_items_cap = 0;                // their number (0: no big leaf)
+    int64_t p2p_items_cap = 0;                // bound of their number (0: no big leaf)
     // Mutual P2P (each unordered pair of big leaves evaluated once): work
     // items of kP2PMutualItem targets, and the source-side sums that a leaf
     // receives from the items of its big backward neighbours (slots 13..25):
@@ -163,6 +162,7 @@ struct Context {
     int64_t cpart_units = 0;                  // entries in use
     DevBuf d_m2l;                             // int32 [cells of levels 2..h-1][189]
     int64_t m2l_off[kMaxLevels] = {0};        // offset (in cells) of a level in d_m2l
+    bool order_built = false;                 // d_order and d_pcount belong to this tree (ensure_parity_order)
     DevBuf d_order;                           // int32 parity-sorted cell index per level (same offsets as d_m2l)
     DevBuf d_pcount;                          // int32 [levels][8]
     DevBuf d_dense;                           // int32 Morton -> cell index tables (levels <= 8)
@@ -282,7 +282,9 @@ inline int32_t* p2p_mutual_next(Context* c) { return reinterpret_cast<int32_t*>(
 // Builds the mutual P2P's work items and slot tables on a built tree and sizes
 // the partial buffer; leaves c->p2p_mutual false when the
 // partial sums would exceed a quarter of the free device memory.
-int build_p2p_mutual_tables(Context* c);
+int build_p2p_mutual_tables(Context* c, int64_t nbig);  // nbig: big leaves
+// The parity order of the cells (d_order, d_pcount) of the built tree.
+int ensure_parity_order(Context* c);
 
 // FP64 passes (fmm_device.hip)
 int run_p2m(Context* c);

@@ -69,29 +69,28 @@ struct KeyIndex {
     }
 };
 
-__global__ __launch_bounds__(256) void k_dense_index(int n, const uint64_t* __restrict__ keys,
-                                                    int32_t* __restrict__ dense) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) dense[keys[i]] = i;
-}
-
 // ---------------------------------------------------------------------------
 // Exclusive scan (three passes: tile sums, scan of tile sums, tile scans).
 template <typename T>
 __device__ T block_exclusive_scan(T v, T* sh, T& total) {
-    const int t = threadIdx.x;
-    sh[t] = v;
-    __syncthreads();
-    for (int d = 1; d < kBlock; d <<= 1) {
-        const T add = t >= d ? sh[t - d] : T(0);
-        __syncthreads();
-        sh[t] += add;
-        __syncthreads();
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    T incl = v;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const T add = __shfl_up(incl, d);
+        if (lane >= d) incl += add;
     }
-    total = sh[kBlock - 1];
-    const T incl = sh[t];
+    if (lane == 63) sh[wave] = incl;
     __syncthreads();
-    return incl - v;
+    T before = 0, sum = 0;
+#pragma unroll
+    for (int w = 0; w < kBlock / 64; ++w) {
+        if (w < wave) before += sh[w];
+        sum += sh[w];
+    }
+    __syncthreads();  // sh may be written again
+    total = sum;
+    return before + incl - v;
 }
 
 template <typename T>
@@ -147,6 +146,33 @@ __global__ __launch_bounds__(kBlock) void k_scan_apply(const T* in, T* out, int6
     }
 }
 
+// The whole scan by one workgroup: for few tiles the launches of the other
+// kernels cost more than the loop over them (about 2 us each).
+constexpr int64_t kScanOneTiles = 8;
+
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_scan_one(const T* in, T* out, int64_t n, T* __restrict__ total_out) {
+    __shared__ T sh[kBlock];
+    T carry = 0;
+    for (int64_t c0 = 0; c0 < n; c0 += kTile) {
+        const int64_t base = c0 + threadIdx.x * kItems;
+        T v[kItems];
+        T s = 0;
+        for (int i = 0; i < kItems; ++i) {
+            v[i] = base + i < n ? in[base + i] : T(0);
+            s += v[i];
+        }
+        T tot;
+        T ex = block_exclusive_scan<T>(s, sh, tot) + carry;
+        for (int i = 0; i < kItems; ++i) {
+            if (base + i < n) out[base + i] = ex;
+            ex += v[i];
+        }
+        carry += tot;
+    }
+    if (threadIdx.x == 0) *total_out = carry;
+}
+
 // out = exclusive scan of in (may alias); *total_dev = sum.
 template <typename T>
 int exclusive_scan(Context* c, const T* in, T* out, int64_t n, T* total_dev, const char* tag) {
@@ -155,6 +181,12 @@ int exclusive_scan(Context* c, const T* in, T* out, int64_t n, T* total_dev, con
         return HFMM_OK;
     }
     const int64_t tiles = (n + kTile - 1) / kTile;
+    if (tiles <= kScanOneTiles) {
+        prof_begin(c, tag);
+        hipLaunchKernelGGL(k_scan_one<T>, dim3(1), dim3(kBlock), 0, c->stream, in, out, n, total_dev);
+        prof_end(c);
+        return check_launch(c, tag);
+    }
     HFMM_TRY(ensure(c, c->d_scan_part, sizeof(T) * static_cast<size_t>(tiles + 1)));
     T* part = c->d_scan_part.as<T>();
     prof_begin(c, tag);
@@ -231,9 +263,11 @@ __global__ __launch_bounds__(kBlock) void k_radix_scatter(const uint64_t* __rest
     }
 }
 
-// Sorts (keys, vals) in place by the low `nbits` bits of the keys, using the
-// context's second key/value buffers; the result ends in keys/vals.
-int radix_sort(Context* c, uint64_t* keys, int32_t* vals, uint64_t* keys2, int32_t* vals2, int64_t n, int nbits) {
+// Sorts (keys, vals) by the low `nbits` bits of the keys, using the second
+// buffers; `swapped`: the result ends in keys2 / vals2.
+int radix_sort(Context* c, uint64_t* keys, int32_t* vals, uint64_t* keys2, int32_t* vals2, int64_t n, int nbits,
+               bool& swapped) {
+    swapped = false;
     if (n <= 1) return HFMM_OK;
     const int64_t ntiles = (n + kTile - 1) / kTile;
     HFMM_TRY(ensure(c, c->d_hist, sizeof(int32_t) * static_cast<size_t>(256 * ntiles + 1)));
@@ -258,10 +292,7 @@ int radix_sort(Context* c, uint64_t* keys, int32_t* vals, uint64_t* keys2, int32
         std::swap(ka, kb);
         std::swap(va, vb);
     }
-    if (ka != keys) {
-        HFMM_HIP(c, hipMemcpyAsync(keys, ka, sizeof(uint64_t) * n, hipMemcpyDeviceToDevice, c->stream));
-        HFMM_HIP(c, hipMemcpyAsync(vals, va, sizeof(int32_t) * n, hipMemcpyDeviceToDevice, c->stream));
-    }
+    swapped = ka != keys;
     return HFMM_OK;
 }
 
@@ -301,21 +332,16 @@ __global__ __launch_bounds__(kBlock) void k_morton(int64_t n, const double* __re
     vals[i] = static_cast<int32_t>(i);
 }
 
-// The inverse of the sort permutation: input index -> sorted index.
-__global__ __launch_bounds__(kBlock) void k_invert_perm(int64_t n, const int32_t* __restrict__ perm,
-                                                       int32_t* __restrict__ iperm) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    iperm[perm[i]] = static_cast<int32_t>(i);
-}
-
+// The sorted particles, and the inverse of the sort permutation (input index ->
+// sorted index), through which the results go back to the input order.
 __global__ __launch_bounds__(kBlock) void k_gather_particles(int64_t n, const int32_t* __restrict__ idx,
                                                             const double* __restrict__ x, const double* __restrict__ y,
                                                             const double* __restrict__ z, const double* __restrict__ q,
-                                                            double* __restrict__ out) {
+                                                            double* __restrict__ out, int32_t* __restrict__ iperm) {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const int32_t o = idx[i];
+    iperm[o] = static_cast<int32_t>(i);
     out[i] = x[o];
     out[n + i] = y[o];
     out[2 * n + i] = z[o];
@@ -342,104 +368,291 @@ __global__ __launch_bounds__(kBlock) void k_gather_charge_chunk(int64_t n, const
     for (int r = 0; r < R; ++r) out[i * R + r] = static_cast<T>(q[static_cast<int64_t>(r0 + r) * n + o]);
 }
 
-// flags[i] = 1 where (keys[i] >> shift) starts a new group.
-__global__ __launch_bounds__(kBlock) void k_head_flags(int64_t n, const uint64_t* __restrict__ keys, int shift,
-                                                      int32_t* __restrict__ flags) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    flags[i] = (i == 0 || (keys[i] >> shift) != (keys[i - 1] >> shift)) ? 1 : 0;
+// The cells of every level from the sorted particle keys at once: particle i
+// begins a cell of level l where its key differs from the one before it in the
+// bits above the levels below l.  k_level_counts counts the cells per tile and
+// level (and the leaves of more than kP2PBig particles: key i + kP2PBig is the
+// same), k_level_scan scans the tiles of each level, k_level_cells writes.  Level
+// by level (flags, scan, write, the count to the host) a tree of height 5 took 24
+// launches and 4 waits.
+struct TreeLevels {
+    int top, leaf;                    // first and last level
+    int64_t lvl_off[kMaxLevels + 1];  // cells before each level
+    int64_t cs_off[kMaxLevels];       // child ranges of each level
+    int64_t ncell[kMaxLevels];
+};
+
+// The highest level at which i begins a cell (leaf + 1: none).
+__device__ __forceinline__ int head_level(uint64_t key, uint64_t before, int64_t i, int top, int leaf) {
+    if (i == 0) return top;
+    const uint64_t d = key ^ before;
+    if (d == 0) return leaf + 1;
+    return max(top, leaf - (63 - __clzll(d)) / 3);
 }
 
-// Writes one entry per group: key >> shift and the index of its first element;
-// group_of[i] (optional) = group of element i.
-__global__ __launch_bounds__(kBlock) void k_write_groups(int64_t n, const uint64_t* __restrict__ keys, int shift,
-                                                        const int32_t* __restrict__ flags,
-                                                        const int32_t* __restrict__ pos, uint64_t* __restrict__ gkey,
-                                                        int32_t* __restrict__ gstart, int32_t* __restrict__ group_of) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int32_t g = pos[i] + flags[i] - 1;
-    if (group_of) group_of[i] = g;
-    if (flags[i]) {
-        gkey[g] = keys[i] >> shift;
-        gstart[g] = static_cast<int32_t>(i);
+__global__ __launch_bounds__(kBlock) void k_level_counts(int64_t n, const uint64_t* __restrict__ keys, int top, int leaf,
+                                                        int64_t ntiles, int32_t* __restrict__ counts,
+                                                        int32_t* __restrict__ nbig) {
+    __shared__ int32_t s[kMaxLevels + 1];
+    if (threadIdx.x <= kMaxLevels) s[threadIdx.x] = 0;
+    __syncthreads();
+    const int64_t base = static_cast<int64_t>(blockIdx.x) * kTile;
+    int big = 0;
+    for (int r = 0; r < kItems; ++r) {
+        const int64_t i = base + r * kBlock + threadIdx.x;
+        if (i >= n) break;
+        const uint64_t key = keys[i];
+        const int h = head_level(key, i ? keys[i - 1] : 0ull, i, top, leaf);
+        if (h > leaf) continue;
+        atomicAdd(&s[h], 1);
+        if (i + kP2PBig < n && keys[i + kP2PBig] == key) ++big;
+    }
+    if (big) atomicAdd(nbig, big);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int sum = 0;  // a cell that begins at level h begins one at every level below
+        for (int l = top; l <= leaf; ++l) {
+            sum += s[l];
+            counts[static_cast<int64_t>(l - top) * ntiles + blockIdx.x] = sum;
+        }
     }
 }
 
-__global__ void k_set_int(int32_t* p, int32_t v) { *p = v; }
-
-// P2P neighbour slots of every leaf: 26 slots in ascending position order,
-// slot -> leaf index or -1 (outside the box or empty).  lim = leaves per axis
-// of one set: the range test is on the set-local coordinates (the low bits),
-// so no list leaves the set of its cell.
-__global__ __launch_bounds__(kBlock) void k_p2p_slots(KeyIndex ix, int lim, int32_t* __restrict__ slots) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int nleaf = ix.n;
-    if (i >= nleaf) return;
-    int x, y, z;
-    demorton3(ix.keys[i], x, y, z);
-    const int lx = x & (lim - 1), ly = y & (lim - 1), lz = z & (lim - 1);
-    int s = 0;
-    for (int dx = -1; dx <= 1; ++dx)
-        for (int dy = -1; dy <= 1; ++dy)
-            for (int dz = -1; dz <= 1; ++dz) {
-                if (!dx && !dy && !dz) continue;
-                const int nx = lx + dx, ny = ly + dy, nz = lz + dz;
-                int f = -1;
-                if (nx >= 0 && nx < lim && ny >= 0 && ny < lim && nz >= 0 && nz < lim)
-                    f = ix.find(morton3(x + dx, y + dy, z + dz));
-                slots[static_cast<int64_t>(i) * kNbrSlots + s] = f;
-                ++s;
-            }
+// One workgroup per level: exclusive scan of its tiles, the sum to total[level].
+__global__ __launch_bounds__(kBlock) void k_level_scan(int64_t ntiles, int32_t* __restrict__ counts,
+                                                      int32_t* __restrict__ total) {
+    __shared__ int32_t sh[kBlock];
+    int32_t* c = counts + static_cast<int64_t>(blockIdx.x) * ntiles;
+    int32_t carry = 0;
+    for (int64_t c0 = 0; c0 < ntiles; c0 += kTile) {
+        const int64_t base = c0 + threadIdx.x * kItems;
+        int32_t v[kItems], sum = 0;
+        for (int i = 0; i < kItems; ++i) {
+            v[i] = base + i < ntiles ? c[base + i] : 0;
+            sum += v[i];
+        }
+        int32_t tot;
+        int32_t ex = block_exclusive_scan<int32_t>(sum, sh, tot) + carry;
+        for (int i = 0; i < kItems; ++i) {
+            if (base + i < ntiles) c[base + i] = ex;
+            ex += v[i];
+        }
+        carry += tot;
+    }
+    if (threadIdx.x == 0) total[blockIdx.x] = carry;
 }
 
-// M2L slots of every cell of a level: 189 slots in the reference enumeration
-// order (parent neighbour x,y,z from -1 to 1, then cousin 0..7, keeping the
-// non-adjacent ones); slot -> cell index in the level or -1.  plim = parents
-// per axis of one set (the range test is set-local, as for the P2P slots).
-__global__ __launch_bounds__(kBlock) void k_m2l_slots(KeyIndex ix, int plim, int32_t* __restrict__ slots) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= ix.n) return;
-    int x, y, z;
-    demorton3(ix.keys[i], x, y, z);
-    const int px = x >> 1, py = y >> 1, pz = z >> 1;
-    const int lx = px & (plim - 1), ly = py & (plim - 1), lz = pz & (plim - 1);
-    const int bx = x & 1, by = y & 1, bz = z & 1;
-    int s = 0;
-    for (int dx = -1; dx <= 1; ++dx)
-        for (int dy = -1; dy <= 1; ++dy)
-            for (int dz = -1; dz <= 1; ++dz) {
-                if (!dx && !dy && !dz) continue;
-                const int ox = lx + dx, oy = ly + dy, oz = lz + dz;
-                const bool inside = ox >= 0 && ox < plim && oy >= 0 && oy < plim && oz >= 0 && oz < plim;
-                const uint64_t pk = inside ? morton3(px + dx, py + dy, pz + dz) : 0ull;
-                for (int cz = 0; cz < 8; ++cz) {
-                    const int xd = 2 * dx + ((cz >> 2) & 1) - bx;
-                    const int yd = 2 * dy + ((cz >> 1) & 1) - by;
-                    const int zd = 2 * dz + (cz & 1) - bz;
-                    if (abs(xd) <= 1 && abs(yd) <= 1 && abs(zd) <= 1) continue;
-                    slots[static_cast<int64_t>(i) * kFarSlots + s] =
-                        inside ? ix.find((pk << 3) | static_cast<uint64_t>(cz)) : -1;
-                    ++s;
-                }
+__global__ __launch_bounds__(kBlock) void k_level_cells(int64_t n, const uint64_t* __restrict__ keys, TreeLevels lv,
+                                                       int64_t ntiles, const int32_t* __restrict__ counts,
+                                                       uint64_t* __restrict__ cellkey, int32_t* __restrict__ cstart,
+                                                       int32_t* __restrict__ lstart, int32_t* __restrict__ pleaf) {
+    __shared__ int32_t sh[kBlock];
+    const int64_t base = static_cast<int64_t>(blockIdx.x) * kTile + threadIdx.x * kItems;
+    uint64_t key[kItems];
+    int head[kItems];
+    for (int i = 0; i < kItems; ++i) {
+        key[i] = 0;
+        head[i] = lv.leaf + 1;
+        if (base + i >= n) continue;
+        key[i] = keys[base + i];
+        const uint64_t before = i ? key[i - 1] : base ? keys[base - 1] : 0ull;
+        head[i] = head_level(key[i], before, base + i, lv.top, lv.leaf);
+    }
+    int32_t below[kItems];  // index of each particle's cell in the level below
+    for (int l = lv.leaf; l >= lv.top; --l) {
+        int32_t sum = 0;
+        for (int i = 0; i < kItems; ++i) sum += head[i] <= l;
+        int32_t tot;
+        int32_t at = block_exclusive_scan<int32_t>(sum, sh, tot) +
+                     counts[static_cast<int64_t>(l - lv.top) * ntiles + blockIdx.x] - 1;
+        for (int i = 0; i < kItems; ++i) {
+            if (base + i >= n) break;
+            if (head[i] <= l) {
+                ++at;
+                cellkey[lv.lvl_off[l] + at] = key[i] >> (3 * (lv.leaf - l));
+                if (l == lv.leaf) lstart[at] = static_cast<int32_t>(base + i);
+                else cstart[lv.cs_off[l] + at] = below[i];
             }
+            if (l == lv.leaf) pleaf[base + i] = at;
+            below[i] = at;
+        }
+    }
+    // the ends of the ranges
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        lstart[lv.ncell[lv.leaf]] = static_cast<int32_t>(n);
+        for (int l = lv.leaf - 1; l >= lv.top; --l)
+            cstart[lv.cs_off[l] + lv.ncell[l]] = static_cast<int32_t>(lv.ncell[l + 1]);
+    }
 }
 
-__global__ __launch_bounds__(kBlock) void k_parity_keys(int ncell, const uint64_t* __restrict__ ckeys,
-                                                       uint64_t* __restrict__ pk, int32_t* __restrict__ idx,
-                                                       int32_t* __restrict__ pcount) {
+// The levels of a launch over cells: level i owns workgroups first[i] ..
+// first[i + 1] - 1, kSlotCells cells each.
+constexpr int kSlotCells = 32;
+struct SlotLevels {
+    int nlev;
+    int first[kMaxLevels + 1];
+    KeyIndex ix[kMaxLevels];
+    int lim[kMaxLevels];  // cells per axis of one set
+    int64_t cell_off[kMaxLevels];
+};
+
+// Morton -> cell tables of the levels that have one.
+__global__ __launch_bounds__(kBlock) void k_dense_index(SlotLevels lv) {
+    const int bid = blockIdx.x;
+    if (bid >= lv.first[lv.nlev]) return;
+    int li = 0;
+    while (bid >= lv.first[li + 1]) ++li;
+    const int i = (bid - lv.first[li]) * kSlotCells + threadIdx.x;
+    if (static_cast<int>(threadIdx.x) < kSlotCells && i < lv.ix[li].n && lv.ix[li].dense)
+        const_cast<int32_t*>(lv.ix[li].dense)[lv.ix[li].keys[i]] = i;
+}
+
+// Slots of every cell of the launch's levels, one entry per thread and turn: the
+// cell at a given offset of each slot (the key by dilated additions on the
+// cell's own, which is decoded once), or -1 where it is empty or outside the set's
+// box.  P2P: the 26 neighbours in position order; M2L: the 189 slots of the cell's
+// parity in the reference enumeration order (offset -> position, slotpos).  A cell
+// at such an offset has its parent beside the cell's, so the box test on the cell
+// is that of the parents.  One thread per cell wrote its slots one by one, 104
+// or 756 bytes from its neighbour's: 163 us for the 262,144 leaves of a 1M tree.
+template <int NSLOT, bool FAR>
+__global__ __launch_bounds__(kBlock) void k_cell_slots(SlotLevels lv, const int16_t* __restrict__ slotpos,
+                                                      int32_t* __restrict__ slots) {
+    constexpr uint64_t MX = 0x4924924924924924ull, MY = 0x2492492492492492ull, MZ = 0x1249249249249249ull;
+    __shared__ uint64_t s_key[kSlotCells];
+    __shared__ int s_pos[kSlotCells][4];  // set-local coordinates, parity
+    __shared__ int16_t s_off[FAR ? 8 * NSLOT : 1];
+    __shared__ uint64_t s_dil[7];
+    const int bid = blockIdx.x;
+    if (bid >= lv.first[lv.nlev]) return;
+    int li = 0;
+    while (bid >= lv.first[li + 1]) ++li;
+    const KeyIndex ix = lv.ix[li];
+    const int lim = lv.lim[li];
+    const int cell0 = (bid - lv.first[li]) * kSlotCells;
+    const int cnt = min(kSlotCells, ix.n - cell0);
+    if (static_cast<int>(threadIdx.x) < cnt) {
+        const uint64_t key = ix.keys[cell0 + threadIdx.x];
+        int x, y, z;
+        demorton3(key, x, y, z);
+        s_key[threadIdx.x] = key;
+        s_pos[threadIdx.x][0] = x & (lim - 1);
+        s_pos[threadIdx.x][1] = y & (lim - 1);
+        s_pos[threadIdx.x][2] = z & (lim - 1);
+        s_pos[threadIdx.x][3] = static_cast<int>(key & 7u);
+    }
+    if (threadIdx.x < 7) s_dil[threadIdx.x] = spread3(static_cast<uint32_t>(static_cast<int>(threadIdx.x) - 3) & 0x1fffffu);
+    if (FAR)
+        for (int i = threadIdx.x; i < 8 * NSLOT; i += kBlock) s_off[i] = slotpos[i];
+    __syncthreads();
+    int32_t* out = slots + (lv.cell_off[li] + cell0) * NSLOT;
+    for (int e = threadIdx.x; e < cnt * NSLOT; e += kBlock) {
+        const int c = e / NSLOT, j = e - c * NSLOT;
+        int dx, dy, dz;
+        if (FAR) {
+            const int pos = s_off[s_pos[c][3] * NSLOT + j];
+            dx = pos / 49 - 3, dy = (pos / 7) % 7 - 3, dz = pos % 7 - 3;
+        } else {
+            const int pos = j < 13 ? j : j + 1;
+            dx = pos / 9 - 1, dy = (pos / 3) % 3 - 1, dz = pos % 3 - 1;
+        }
+        const int nx = s_pos[c][0] + dx, ny = s_pos[c][1] + dy, nz = s_pos[c][2] + dz;
+        int f = -1;
+        if (nx >= 0 && nx < lim && ny >= 0 && ny < lim && nz >= 0 && nz < lim) {
+            const uint64_t key = s_key[c];
+            const uint64_t kx = ((key | ~MX) + (s_dil[dx + 3] << 2)) & MX;
+            const uint64_t ky = ((key | ~MY) + (s_dil[dy + 3] << 1)) & MY;
+            const uint64_t kz = ((key | ~MZ) + s_dil[dz + 3]) & MZ;
+            f = ix.find(kx | ky | kz);
+        }
+        out[e] = f;
+    }
+}
+
+// Cells of a level grouped by child index (stable), every level in one launch:
+// per tile of kTile cells the counts of the 8 parities, their scan over the
+// tiles of the level, parity by parity, and the places.  Eight 16-bit counters
+// in two words.
+struct ParityLevels {
+    int nlev;
+    int first[kMaxLevels + 1];  // tiles before each level
+    int64_t cell_off[kMaxLevels];
+    int ncell[kMaxLevels];
+    int level[kMaxLevels];
+};
+
+__global__ __launch_bounds__(kBlock) void k_parity_counts(ParityLevels lv, const uint64_t* __restrict__ cellkey,
+                                                         int32_t* __restrict__ counts) {
     __shared__ int32_t s[8];
+    int li = 0;
+    while (static_cast<int>(blockIdx.x) >= lv.first[li + 1]) ++li;
     if (threadIdx.x < 8) s[threadIdx.x] = 0;
     __syncthreads();
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < ncell) {
-        const int par = static_cast<int>(ckeys[i] & 7u);
-        pk[i] = static_cast<uint64_t>(par);
-        idx[i] = i;
-        atomicAdd(&s[par], 1);
+    const int base = (static_cast<int>(blockIdx.x) - lv.first[li]) * kTile;
+    for (int r = 0; r < kItems; ++r) {
+        const int i = base + r * kBlock + static_cast<int>(threadIdx.x);
+        if (i < lv.ncell[li]) atomicAdd(&s[cellkey[lv.cell_off[li] + i] & 7u], 1);
     }
     __syncthreads();
-    if (threadIdx.x < 8 && s[threadIdx.x]) atomicAdd(&pcount[threadIdx.x], s[threadIdx.x]);
+    if (threadIdx.x < 8) counts[blockIdx.x * 8 + threadIdx.x] = s[threadIdx.x];
+}
+
+// One workgroup per level: counts[tile][parity] -> first place of the tile's
+// cells of that parity; pcount[level][parity].
+__global__ __launch_bounds__(64) void k_parity_scan(ParityLevels lv, int32_t* __restrict__ counts,
+                                                   int32_t* __restrict__ pcount) {
+    __shared__ int32_t s_sum[8], s_start[8];
+    const int li = blockIdx.x, lane = threadIdx.x;
+    const int t0 = lv.first[li], t1 = lv.first[li + 1];
+    if (lane < 8) {
+        int sum = 0;
+        for (int t = t0; t < t1; ++t) sum += counts[t * 8 + lane];
+        s_sum[lane] = sum;
+        pcount[8 * lv.level[li] + lane] = sum;
+    }
+    __syncthreads();
+    if (lane == 0) {
+        int run = 0;
+        for (int p = 0; p < 8; ++p) {
+            s_start[p] = run;
+            run += s_sum[p];
+        }
+    }
+    __syncthreads();
+    if (lane < 8) {
+        int run = s_start[lane];
+        for (int t = t0; t < t1; ++t) {
+            const int c = counts[t * 8 + lane];
+            counts[t * 8 + lane] = run;
+            run += c;
+        }
+    }
+}
+
+__global__ __launch_bounds__(kBlock) void k_parity_order(ParityLevels lv, const uint64_t* __restrict__ cellkey,
+                                                        const int32_t* __restrict__ counts, int32_t* __restrict__ order) {
+    __shared__ uint64_t sh[kBlock];
+    int li = 0;
+    while (static_cast<int>(blockIdx.x) >= lv.first[li + 1]) ++li;
+    const int base = (static_cast<int>(blockIdx.x) - lv.first[li]) * kTile + static_cast<int>(threadIdx.x) * kItems;
+    int par[kItems];
+    uint64_t c0 = 0, c1 = 0;
+    for (int i = 0; i < kItems; ++i) {
+        par[i] = base + i < lv.ncell[li] ? static_cast<int>(cellkey[lv.cell_off[li] + base + i] & 7u) : -1;
+        if (par[i] >= 4) c1 += 1ull << (16 * (par[i] - 4));
+        else if (par[i] >= 0) c0 += 1ull << (16 * par[i]);
+    }
+    uint64_t tot;
+    uint64_t e0 = block_exclusive_scan<uint64_t>(c0, sh, tot);
+    uint64_t e1 = block_exclusive_scan<uint64_t>(c1, sh, tot);
+    for (int i = 0; i < kItems; ++i) {
+        if (par[i] < 0) break;
+        uint64_t& e = par[i] >= 4 ? e1 : e0;
+        const int sft = 16 * (par[i] & 3);
+        const int at = counts[blockIdx.x * 8 + par[i]] + static_cast<int>((e >> sft) & 0xffffu);
+        e += 1ull << sft;
+        order[lv.cell_off[li] + at] = base + i;
+    }
 }
 
 inline unsigned blocks_for(int64_t n) { return static_cast<unsigned>((n + kBlock - 1) / kBlock); }
@@ -462,8 +675,6 @@ __global__ __launch_bounds__(kBlock) void k_m2l_slot_counts(int ncell, const uin
         if (bins[j]) atomicAdd(&counts[j], static_cast<unsigned long long>(bins[j]));
 }
 
-// Run-length groups of sorted keys >> shift: writes group keys and starts,
-// returns the count on the host.
 // P2P work items of the big leaves: ceil(count / kP2PItem) items of
 // consecutive targets per leaf with more than kP2PBig particles.
 template <int ITEM>
@@ -544,7 +755,9 @@ int sort_p2p_items(Context* c, int2* items, const int32_t* nitems, int64_t cap) 
                        items, c->d_leafstart.as<int32_t>(), c->d_p2p.as<int32_t>(), ik, iv);
     prof_end(c);
     HFMM_TRY(check_launch(c, "p2p_items"));
-    HFMM_TRY(radix_sort(c, ik, iv, ik + cap, iv + cap, cap, 32));
+    bool swapped = false;
+    HFMM_TRY(radix_sort(c, ik, iv, ik + cap, iv + cap, cap, 32, swapped));
+    if (swapped) iv += cap;
     HFMM_HIP(c, hipMemcpyAsync(c->d_items_tmp.ptr, items, sizeof(int2) * static_cast<size_t>(cap),
                                hipMemcpyDeviceToDevice, c->stream));
     prof_begin(c, "p2p_items");
@@ -603,30 +816,6 @@ __global__ __launch_bounds__(kBlock) void k_colslot_counts(int nleaf, const int3
     units[i] = static_cast<int64_t>(run + k - 1) * m;
 }
 
-int make_groups(Context* c, const uint64_t* keys, int64_t n, int shift, uint64_t* gkey, int32_t* gstart,
-                int32_t* group_of, int64_t& count, const char* tag) {
-    HFMM_TRY(ensure(c, c->d_flags, sizeof(int32_t) * static_cast<size_t>(n + 1)));
-    HFMM_TRY(ensure(c, c->d_scan, sizeof(int32_t) * static_cast<size_t>(n + 1)));
-    int32_t* flags = c->d_flags.as<int32_t>();
-    int32_t* pos = c->d_scan.as<int32_t>();
-    int32_t* total = reinterpret_cast<int32_t*>(c->d_count.as<int64_t>() + 14);
-    prof_begin(c, tag);
-    hipLaunchKernelGGL(k_head_flags, dim3(blocks_for(n)), dim3(kBlock), 0, c->stream, n, keys, shift, flags);
-    prof_end(c);
-    HFMM_TRY(check_launch(c, tag));
-    HFMM_TRY(exclusive_scan<int32_t>(c, flags, pos, n, total, "group_scan"));
-    prof_begin(c, tag);
-    hipLaunchKernelGGL(k_write_groups, dim3(blocks_for(n)), dim3(kBlock), 0, c->stream, n, keys, shift, flags, pos,
-                       gkey, gstart, group_of);
-    prof_end(c);
-    HFMM_TRY(check_launch(c, tag));
-    int32_t h_total = 0;
-    HFMM_HIP(c, hipMemcpyAsync(&h_total, total, sizeof(int32_t), hipMemcpyDeviceToHost, c->stream));
-    HFMM_HIP(c, hipStreamSynchronize(c->stream));
-    count = h_total;
-    return HFMM_OK;
-}
-
 }  // namespace
 
 int m2l_slot_counts(Context* c, int level, unsigned long long* counts) {
@@ -678,13 +867,13 @@ int build_tree_device(Context* c) {
     if (n > (int64_t(1) << 30)) return fail(c, HFMM_ERR_ARG, "more than 2^30 particles");
     HFMM_TRY(ensure(c, c->d_keys, sizeof(uint64_t) * n));
     HFMM_TRY(ensure(c, c->d_keys2, sizeof(uint64_t) * n));
-    HFMM_TRY(ensure(c, c->d_vals, sizeof(int32_t) * n));
+    HFMM_TRY(ensure(c, c->d_perm, sizeof(int32_t) * n));
     HFMM_TRY(ensure(c, c->d_vals2, sizeof(int32_t) * n));
     HFMM_TRY(ensure(c, c->d_count, sizeof(int64_t) * 24));
-    uint64_t* keys = c->d_keys.as<uint64_t>();
-    int32_t* vals = c->d_vals.as<int32_t>();
-    int32_t* err = reinterpret_cast<int32_t*>(c->d_count.as<int64_t>() + 13);
-    HFMM_HIP(c, hipMemsetAsync(err, 0, sizeof(int32_t), c->stream));
+    // what the host reads once: the error flag, the big leaves, the cells of each level
+    HFMM_TRY(ensure(c, c->d_flags, sizeof(int32_t) * (2 + kMaxLevels)));
+    int32_t* info = c->d_flags.as<int32_t>();
+    HFMM_HIP(c, hipMemsetAsync(info, 0, sizeof(int32_t) * 2, c->stream));
 
     // 1. keys (boxCorner = center + (-(width/2)), FGroupTree.hpp:183)
     const double half = c->P.box_width / 2;
@@ -693,108 +882,123 @@ int build_tree_device(Context* c) {
     hipLaunchKernelGGL(k_morton, dim3(blocks_for(n)), dim3(kBlock), 0, c->stream, n, c->x, c->y, c->z,
                        c->P.box_center[0] + (-half), c->P.box_center[1] + (-half), c->P.box_center[2] + (-half),
                        c->P.box_width, leafw, Lloc, c->nsets > 1 ? c->d_setoff.as<int64_t>() : nullptr, c->nsets,
-                       keys, vals, err);
+                       c->d_keys.as<uint64_t>(), c->d_perm.as<int32_t>(), info);
     prof_end(c);
     HFMM_TRY(check_launch(c, "morton"));
-    int32_t h_err = 0;
-    HFMM_HIP(c, hipMemcpyAsync(&h_err, err, sizeof(int32_t), hipMemcpyDeviceToHost, c->stream));
-    HFMM_HIP(c, hipStreamSynchronize(c->stream));
-    if (h_err) return fail(c, HFMM_ERR_OUTSIDE_BOX, "a particle lies outside the simulation box");
 
     // 2. stable sort by key (ties keep the input order)
-    HFMM_TRY(radix_sort(c, keys, vals, c->d_keys2.as<uint64_t>(), c->d_vals2.as<int32_t>(), n, 3 * L));
-
-    // 3. sorted particle SoA
-    // kSortedPad doubles after the four SoA arrays: the big-leaf P2P reads whole
-    // blocks of sources past a leaf's end (and masks them)
-    HFMM_TRY(ensure(c, c->d_sorted, sizeof(double) * (4 * n + kSortedPad)));
-    HFMM_TRY(ensure(c, c->d_perm, sizeof(int32_t) * n));
-    HFMM_HIP(c, hipMemcpyAsync(c->d_perm.ptr, vals, sizeof(int32_t) * n, hipMemcpyDeviceToDevice, c->stream));
-    // the results are written back in input order through the inverse
-    HFMM_TRY(ensure(c, c->d_iperm, sizeof(int32_t) * n));
-    hipLaunchKernelGGL(k_invert_perm, dim3(blocks_for(n)), dim3(kBlock), 0, c->stream, n, vals,
-                       c->d_iperm.as<int32_t>());
-    HFMM_TRY(check_launch(c, "invert_perm"));
-    prof_begin(c, "gather");
-    hipLaunchKernelGGL(k_gather_particles, dim3(blocks_for(n)), dim3(kBlock), 0, c->stream, n, vals, c->x, c->y, c->z,
-                       c->q, c->d_sorted.as<double>());
-    prof_end(c);
-    HFMM_TRY(check_launch(c, "gather"));
-
-    // 4. leaves, then the parent levels down to 2; the cell keys of every level
-    // are first produced into a per-level scratch table of capacity n.
-    const int64_t cap = n;
-    HFMM_TRY(ensure(c, c->d_cellkey_tmp, sizeof(uint64_t) * static_cast<size_t>(cap) * h));
-    HFMM_TRY(ensure(c, c->d_leafstart, sizeof(int32_t) * (n + 1)));
-    HFMM_TRY(ensure(c, c->d_pleaf, sizeof(int32_t) * n));
-    // child-start table: per level ncell+1 entries, at most cap+1 each
-    HFMM_TRY(ensure(c, c->d_childstart, sizeof(int32_t) * static_cast<size_t>(cap + 1) * h));
-    uint64_t* tkeys = c->d_cellkey_tmp.as<uint64_t>();
-    int32_t* cstart = c->d_childstart.as<int32_t>();
-    for (int l = 0; l < kMaxLevels; ++l) c->ncell[l] = 0;
-    int64_t nl = 0;
-    HFMM_TRY(make_groups(c, keys, n, 0, tkeys + static_cast<size_t>(L) * cap, c->d_leafstart.as<int32_t>(),
-                         c->d_pleaf.as<int32_t>(), nl, "leaves"));
-    c->ncell[L] = nl;
-    hipLaunchKernelGGL(k_set_int, dim3(1), dim3(1), 0, c->stream, c->d_leafstart.as<int32_t>() + nl,
-                       static_cast<int32_t>(n));
-    for (int l = L - 1; l >= top; --l) {
-        int64_t np = 0;
-        int32_t* cs = cstart + static_cast<size_t>(l) * (cap + 1);
-        HFMM_TRY(make_groups(c, tkeys + static_cast<size_t>(l + 1) * cap, c->ncell[l + 1], 3,
-                             tkeys + static_cast<size_t>(l) * cap, cs, nullptr, np, "levels"));
-        c->ncell[l] = np;
-        hipLaunchKernelGGL(k_set_int, dim3(1), dim3(1), 0, c->stream, cs + np, static_cast<int32_t>(c->ncell[l + 1]));
-        c->cs_off[l] = static_cast<int64_t>(l) * (cap + 1);
+    bool swapped = false;
+    HFMM_TRY(radix_sort(c, c->d_keys.as<uint64_t>(), c->d_perm.as<int32_t>(), c->d_keys2.as<uint64_t>(),
+                        c->d_vals2.as<int32_t>(), n, 3 * L, swapped));
+    if (swapped) {
+        std::swap(c->d_keys, c->d_keys2);
+        std::swap(c->d_perm, c->d_vals2);
     }
-    // pack the cell keys of levels top..h-1 contiguously
-    int64_t off = 0;
+    const uint64_t* keys = c->d_keys.as<uint64_t>();
+
+    // 3. cells per level, and on the host
+    const int64_t ntiles = (n + kTile - 1) / kTile;
+    HFMM_TRY(ensure(c, c->d_scan_part, sizeof(int32_t) * static_cast<size_t>(ntiles) * (L - top + 1)));
+    int32_t* counts = c->d_scan_part.as<int32_t>();
+    prof_begin(c, "levels");
+    hipLaunchKernelGGL(k_level_counts, dim3(static_cast<unsigned>(ntiles)), dim3(kBlock), 0, c->stream, n, keys, top, L,
+                       ntiles, counts, info + 1);
+    hipLaunchKernelGGL(k_level_scan, dim3(L - top + 1), dim3(kBlock), 0, c->stream, ntiles, counts, info + 2);
+    prof_end(c);
+    HFMM_TRY(check_launch(c, "levels"));
+    int32_t h_info[2 + kMaxLevels] = {0};
+    HFMM_HIP(c, hipMemcpyAsync(h_info, info, sizeof(int32_t) * (2 + L - top + 1), hipMemcpyDeviceToHost, c->stream));
+    HFMM_HIP(c, hipStreamSynchronize(c->stream));
+    if (h_info[0]) return fail(c, HFMM_ERR_OUTSIDE_BOX, "a particle lies outside the simulation box");
+    TreeLevels lv{};
+    lv.top = top;
+    lv.leaf = L;
+    int64_t off = 0, cs = 0;
+    for (int l = 0; l < kMaxLevels; ++l) c->ncell[l] = 0;
     for (int l = 0; l <= L; ++l) {
-        c->lvl_off[l] = off;
-        if (l >= top) off += c->ncell[l];
+        c->lvl_off[l] = c->m2l_off[l] = lv.lvl_off[l] = off;
+        if (l < top) continue;
+        c->ncell[l] = lv.ncell[l] = h_info[2 + l - top];
+        off += c->ncell[l];
+        c->cs_off[l] = lv.cs_off[l] = cs;
+        cs += c->ncell[l] + 1;
     }
     c->lvl_off[L + 1] = off;
     c->total_cells = off;
-    HFMM_TRY(ensure(c, c->d_cellkey, sizeof(uint64_t) * static_cast<size_t>(off)));
-    for (int l = top; l <= L; ++l)
-        HFMM_HIP(c, hipMemcpyAsync(c->d_cellkey.as<uint64_t>() + c->lvl_off[l], tkeys + static_cast<size_t>(l) * cap,
-                                   sizeof(uint64_t) * c->ncell[l], hipMemcpyDeviceToDevice, c->stream));
+    const int64_t nl = c->ncell[L];
 
-    // dense Morton -> cell tables for the levels with at most 2^24 cells
+    // 4. sorted particle SoA
+    // kSortedPad doubles after the four SoA arrays: the big-leaf P2P reads whole
+    // blocks of sources past a leaf's end (and masks them)
+    HFMM_TRY(ensure(c, c->d_sorted, sizeof(double) * (4 * n + kSortedPad)));
+    HFMM_TRY(ensure(c, c->d_iperm, sizeof(int32_t) * n));
+    prof_begin(c, "gather");
+    hipLaunchKernelGGL(k_gather_particles, dim3(blocks_for(n)), dim3(kBlock), 0, c->stream, n, c->d_perm.as<int32_t>(),
+                       c->x, c->y, c->z, c->q, c->d_sorted.as<double>(), c->d_iperm.as<int32_t>());
+    prof_end(c);
+    HFMM_TRY(check_launch(c, "gather"));
+
+    // 5. cell keys, leaf and child ranges
+    HFMM_TRY(ensure(c, c->d_cellkey, sizeof(uint64_t) * static_cast<size_t>(off)));
+    HFMM_TRY(ensure(c, c->d_leafstart, sizeof(int32_t) * (nl + 1)));
+    HFMM_TRY(ensure(c, c->d_pleaf, sizeof(int32_t) * n));
+    HFMM_TRY(ensure(c, c->d_childstart, sizeof(int32_t) * static_cast<size_t>(cs)));
+    prof_begin(c, "levels");
+    hipLaunchKernelGGL(k_level_cells, dim3(static_cast<unsigned>(ntiles)), dim3(kBlock), 0, c->stream, n, keys, lv,
+                       ntiles, counts, c->d_cellkey.as<uint64_t>(), c->d_childstart.as<int32_t>(),
+                       c->d_leafstart.as<int32_t>(), c->d_pleaf.as<int32_t>());
+    prof_end(c);
+    HFMM_TRY(check_launch(c, "levels"));
+
+    // 6. dense Morton -> cell tables for the levels with at most 2^24 cells, then
+    // the P2P slots of the leaves and the M2L slots of levels top..h-1
     int64_t dense_total = 0;
     int64_t dense_off[kMaxLevels];
-    for (int l = 0; l <= L; ++l) {
+    for (int l = top; l <= L; ++l) {
         dense_off[l] = -1;
-        if (l >= top && 3 * l <= 24) {
+        if (3 * l <= 24) {
             dense_off[l] = dense_total;
             dense_total += int64_t(1) << (3 * l);
         }
     }
     HFMM_TRY(ensure(c, c->d_dense, sizeof(int32_t) * static_cast<size_t>(dense_total + 1)));
     HFMM_HIP(c, hipMemsetAsync(c->d_dense.ptr, 0xFF, sizeof(int32_t) * static_cast<size_t>(dense_total), c->stream));
-    KeyIndex ix[kMaxLevels];
+    SlotLevels sl{}, leaf{};
     for (int l = top; l <= L; ++l) {
-        ix[l].keys = c->d_cellkey.as<uint64_t>() + c->lvl_off[l];
-        ix[l].n = static_cast<int>(c->ncell[l]);
-        ix[l].dense = dense_off[l] >= 0 ? c->d_dense.as<int32_t>() + dense_off[l] : nullptr;
-        if (ix[l].dense) {
-            prof_begin(c, "dense_index");
-            hipLaunchKernelGGL(k_dense_index, dim3(blocks_for(c->ncell[l])), dim3(kBlock), 0, c->stream, ix[l].n,
-                               ix[l].keys, c->d_dense.as<int32_t>() + dense_off[l]);
-            prof_end(c);
-            HFMM_TRY(check_launch(c, "dense_index"));
-        }
+        const int i = sl.nlev++;
+        sl.ix[i].keys = c->d_cellkey.as<uint64_t>() + c->lvl_off[l];
+        sl.ix[i].n = static_cast<int>(c->ncell[l]);
+        sl.ix[i].dense = dense_off[l] >= 0 ? c->d_dense.as<int32_t>() + dense_off[l] : nullptr;
+        sl.lim[i] = 1 << (l - c->set_levels);
+        sl.cell_off[i] = c->lvl_off[l];
+        sl.first[i + 1] = sl.first[i] + static_cast<int>((c->ncell[l] + kSlotCells - 1) / kSlotCells);
     }
-
-    // 5. P2P slots of the leaves
+    leaf.nlev = 1;
+    leaf.ix[0] = sl.ix[sl.nlev - 1];
+    leaf.lim[0] = sl.lim[sl.nlev - 1];
+    leaf.first[1] = sl.first[sl.nlev] - sl.first[sl.nlev - 1];
     HFMM_TRY(ensure(c, c->d_p2p, sizeof(int32_t) * static_cast<size_t>(nl) * kNbrSlots));
+    HFMM_TRY(ensure(c, c->d_m2l, sizeof(int32_t) * static_cast<size_t>(off) * kFarSlots));
+    prof_begin(c, "dense_index");
+    hipLaunchKernelGGL(k_dense_index, dim3(sl.first[sl.nlev]), dim3(64), 0, c->stream, sl);
+    prof_end(c);
+    HFMM_TRY(check_launch(c, "dense_index"));
     prof_begin(c, "p2p_lists");
-    hipLaunchKernelGGL(k_p2p_slots, dim3(blocks_for(nl)), dim3(kBlock), 0, c->stream, ix[L], 1 << Lloc,
-                       c->d_p2p.as<int32_t>());
+    hipLaunchKernelGGL((k_cell_slots<kNbrSlots, false>), dim3(leaf.first[1]), dim3(kBlock), 0, c->stream, leaf,
+                       c->d_slotpos.as<int16_t>(), c->d_p2p.as<int32_t>());
     prof_end(c);
     HFMM_TRY(check_launch(c, "p2p_lists"));
-    {
-        // items of the big leaves (slot 12 of d_count: their number)
+    prof_begin(c, "m2l_lists");
+    hipLaunchKernelGGL((k_cell_slots<kFarSlots, true>), dim3(sl.first[sl.nlev]), dim3(kBlock), 0, c->stream, sl,
+                       c->d_slotpos.as<int16_t>(), c->d_m2l.as<int32_t>());
+    prof_end(c);
+    HFMM_TRY(check_launch(c, "m2l_lists"));
+
+    // 7. work items of the big leaves (slot 12 of d_count: their number)
+    const int64_t nbig = h_info[1];
+    c->p2p_items_cap = nbig > 0 ? n / kP2PItem + nbig : 0;
+    if (c->p2p_items_cap > 0) {
+        HFMM_TRY(ensure(c, c->d_p2pitems, sizeof(int2) * static_cast<size_t>(c->p2p_items_cap)));
         HFMM_TRY(ensure(c, c->d_flags, sizeof(int32_t) * static_cast<size_t>(nl + 1)));
         HFMM_TRY(ensure(c, c->d_scan, sizeof(int32_t) * static_cast<size_t>(nl + 1)));
         prof_begin(c, "p2p_items");
@@ -804,13 +1008,6 @@ int build_tree_device(Context* c) {
         HFMM_TRY(check_launch(c, "p2p_items"));
         HFMM_TRY(exclusive_scan<int32_t>(c, c->d_flags.as<int32_t>(), c->d_scan.as<int32_t>(), nl, p2p_item_count(c),
                                          "p2p_items"));
-        int32_t items = 0;
-        HFMM_HIP(c, hipMemcpyAsync(&items, p2p_item_count(c), sizeof(int32_t), hipMemcpyDeviceToHost, c->stream));
-        HFMM_HIP(c, hipStreamSynchronize(c->stream));
-        c->p2p_items_cap = items;
-    }
-    if (c->p2p_items_cap > 0) {
-        HFMM_TRY(ensure(c, c->d_p2pitems, sizeof(int2) * static_cast<size_t>(c->p2p_items_cap)));
         prof_begin(c, "p2p_items");
         hipLaunchKernelGGL(k_p2p_items<kP2PItem>, dim3(blocks_for(nl)), dim3(kBlock), 0, c->stream, static_cast<int>(nl),
                            c->d_leafstart.as<int32_t>(), c->d_scan.as<int32_t>(), c->d_p2pitems.as<int2>());
@@ -820,44 +1017,47 @@ int build_tree_device(Context* c) {
         // first spreads the large ones over the waves
         HFMM_TRY((sort_p2p_items<kP2PItem, false>(c, c->d_p2pitems.as<int2>(), p2p_item_count(c), c->p2p_items_cap)));
     }
-
-    // 6. M2L slots and parity-sorted target order of levels top..h-1
-    HFMM_TRY(ensure(c, c->d_m2l, sizeof(int32_t) * static_cast<size_t>(off) * kFarSlots));
-    HFMM_TRY(ensure(c, c->d_order, sizeof(int32_t) * static_cast<size_t>(off)));
-    HFMM_TRY(ensure(c, c->d_pcount, sizeof(int32_t) * 8 * kMaxLevels));
-    HFMM_HIP(c, hipMemsetAsync(c->d_pcount.ptr, 0, sizeof(int32_t) * 8 * kMaxLevels, c->stream));
-    for (int l = top; l <= L; ++l) {
-        const int64_t nc = c->ncell[l];
-        c->m2l_off[l] = c->lvl_off[l];
-        const uint64_t* ck = c->d_cellkey.as<uint64_t>() + c->lvl_off[l];
-        prof_begin(c, "m2l_lists");
-        hipLaunchKernelGGL(k_m2l_slots, dim3(blocks_for(nc)), dim3(kBlock), 0, c->stream, ix[l],
-                           1 << (l - 1 - c->set_levels),
-                           c->d_m2l.as<int32_t>() + static_cast<size_t>(c->m2l_off[l]) * kFarSlots);
-        prof_end(c);
-        HFMM_TRY(check_launch(c, "m2l_lists"));
-        // parity order: stable sort of (key & 7) carrying the cell index
-        int32_t* ord = c->d_order.as<int32_t>() + c->lvl_off[l];
-        prof_begin(c, "parity");
-        // (the per-level key scratch is free once the keys are packed)
-        hipLaunchKernelGGL(k_parity_keys, dim3(blocks_for(nc)), dim3(kBlock), 0, c->stream, static_cast<int>(nc), ck,
-                           tkeys, ord, c->d_pcount.as<int32_t>() + 8 * l);
-        prof_end(c);
-        HFMM_TRY(check_launch(c, "parity"));
-        HFMM_TRY(radix_sort(c, tkeys, ord, tkeys + cap, c->d_vals2.as<int32_t>(), nc, 3));
-    }
     c->tree_built = true;
     c->evaluated = false;
     c->p2p_mutual = false;
-    if (c->p2p_items_cap > 0) HFMM_TRY(build_p2p_mutual_tables(c));
+    c->order_built = false;
+    if (c->p2p_items_cap > 0) HFMM_TRY(build_p2p_mutual_tables(c, nbig));
+    return is_mixed(c) ? ensure_parity_order(c) : HFMM_OK;
+}
+
+// The cells of every level by child index (mixed and global-SVD M2L; the
+// symmetric FP64 M2L takes them as they are).
+int ensure_parity_order(Context* c) {
+    if (c->order_built) return HFMM_OK;
+    ParityLevels lv{};
+    for (int l = c->top(); l < c->height(); ++l) {
+        const int i = lv.nlev++;
+        lv.cell_off[i] = c->lvl_off[l];
+        lv.ncell[i] = static_cast<int>(c->ncell[l]);
+        lv.level[i] = l;
+        lv.first[i + 1] = lv.first[i] + static_cast<int>((c->ncell[l] + kTile - 1) / kTile);
+    }
+    HFMM_TRY(ensure(c, c->d_order, sizeof(int32_t) * static_cast<size_t>(c->total_cells)));
+    HFMM_TRY(ensure(c, c->d_pcount, sizeof(int32_t) * 8 * kMaxLevels));
+    HFMM_TRY(ensure(c, c->d_hist, sizeof(int32_t) * 8 * static_cast<size_t>(lv.first[lv.nlev])));
+    int32_t* counts = c->d_hist.as<int32_t>();
+    prof_begin(c, "parity");
+    hipLaunchKernelGGL(k_parity_counts, dim3(lv.first[lv.nlev]), dim3(kBlock), 0, c->stream, lv,
+                       c->d_cellkey.as<uint64_t>(), counts);
+    hipLaunchKernelGGL(k_parity_scan, dim3(lv.nlev), dim3(64), 0, c->stream, lv, counts, c->d_pcount.as<int32_t>());
+    hipLaunchKernelGGL(k_parity_order, dim3(lv.first[lv.nlev]), dim3(kBlock), 0, c->stream, lv,
+                       c->d_cellkey.as<uint64_t>(), counts, c->d_order.as<int32_t>());
+    prof_end(c);
+    HFMM_TRY(check_launch(c, "parity"));
+    c->order_built = true;
     return HFMM_OK;
 }
 
-int build_p2p_mutual_tables(Context* c) {
+int build_p2p_mutual_tables(Context* c, int64_t nbig) {
     c->p2p_mutual = false;
     const int64_t nl = c->ncell[c->height() - 1];
     const int32_t* lstart = c->d_leafstart.as<int32_t>();
-    c->p2p_items_m_cap = c->n / kP2PMutualItem + c->n / (kP2PBig + 1) + 1;
+    c->p2p_items_m_cap = c->n / kP2PMutualItem + nbig;
     HFMM_TRY(ensure(c, c->d_p2pitems_m, sizeof(int2) * static_cast<size_t>(c->p2p_items_m_cap)));
     HFMM_TRY(ensure(c, c->d_flags, sizeof(int32_t) * static_cast<size_t>(nl + 1)));
     HFMM_TRY(ensure(c, c->d_scan, sizeof(int32_t) * static_cast<size_t>(nl + 1)));
