@@ -14,10 +14,11 @@ computed by the library's FP64 direct-sum kernel, outside the timed region).
 
 `roofline` is the kernel with the largest share of the step, with its
 algorithmic work over the HIP-event time of its launches in the timed region:
-  - M2L: the reference's flop count 4 p^3 k - k - p^3 per interaction
-    (Src/Kernels/Chebyshev/FChebFlopsSymKernel.hpp:62-63); the mixed form
-    executes it as six bfloat16 partial products, so its algorithmic bf16 work
-    is six times that count, against the bf16 dense MFMA peak;
+  - M2L: the FP64 class products that are executed, against the FP64 MFMA peak
+    (the reference's flop count 4 p^3 k - k - p^3 per interaction,
+    Src/Kernels/Chebyshev/FChebFlopsSymKernel.hpp:62-63, stands beside it); a
+    mixed form's bfloat16 tiles execute that count as six (three) partial
+    products, against the bf16 dense MFMA peak;
   - P2P: 34 flops per target-source pair (FChebFlopsSymKernel.hpp:64-65)
     against the FP32 (mixed) or FP64 vector peak.
 `cpu_baseline` times the FP64 OpenMP oracle on a bounded sample of the same
@@ -115,6 +116,23 @@ def p2p_pairs(engine):
             "big_big": float(big_big), "big_rest": float(per_leaf[big].sum() - big_big)}
 
 
+F64_PRODUCTS = 4  # the mixed forms' M2L variant that runs the FP64 products
+
+
+def executed_m2l_flops(engine, order):
+    """FP64 flops of the class products (csrc/m2l_f64.hip): per cell two
+    products of p^3 nodes with the ranks of the 56 offsets that differ in more
+    than signs (tiles without an offset skip it, which is not counted)."""
+    rows = 0
+    for x in range(4):
+        for y in range(4):
+            for z in range(4):
+                if max(x, y, z) > 1:
+                    rows += engine.operator(_canonical(x, y, z))[0].shape[1]
+    cells = sum(engine.tree_info().n_cells)
+    return 4.0 * order ** 3 * rows * cells
+
+
 def make_particles(dist, n):
     from scalfmm_amd.distributions import plummer, uniform_cube
     return (plummer if dist == "plummer" else uniform_cube)(n, SEED[dist])
@@ -138,7 +156,7 @@ def cpu_baseline(dist, n, h, p):
 # only while that file is unchanged (its sha256 is recorded in the summary)
 KERNEL_SOURCE = {
     "k_p2p_mixed_big": "p2p_mixed.hip", "k_p2p_mixed_mutual": "p2p_mixed.hip", "k_m2l_mixed": "fmm_mixed.hip",
-    "k_p2p_mixed": "p2p_mixed.hip", "k_m2l_f64": "fmm_device.hip", "k_p2p_f64_big": "fmm_device.hip",
+    "k_p2p_mixed": "p2p_mixed.hip", "k_m2l_up": "m2l_f64.hip", "k_p2p_f64_mutual": "fmm_device.hip",
     "k_p2p_f64": "fmm_device.hip", "k_unif_m2l": "fmm_global.hip",
 }
 
@@ -234,6 +252,10 @@ DTYPE = {"mixed": "bf16x3-mfma/f32 (M2L), f32 (P2P), f64 (rest)",
          "hilo": "bf16x2-mfma/f32 (M2L), f32 (P2P), f64 (rest)", "fp64": "f64"}
 
 
+def dtype_of(form, m2l_variant):
+    return "f64 (M2L), f32 (P2P), f64 (rest)" if form != "fp64" and m2l_variant == F64_PRODUCTS else DTYPE[form]
+
+
 def precision_code(form):
     from scalfmm_amd import _abi
     return {"mixed": _abi.PRECISION_MIXED, "hilo": _abi.PRECISION_MIXED_HILO, "fp64": _abi.PRECISION_FP64}[form]
@@ -254,11 +276,16 @@ def roofline(engines, kernel_ms, launches, p, form, workload, nrhs=1, kernel=Non
             f, c = algorithmic_m2l_flops(e, e.height, p)
             flops += f * nrhs
             n_int += c * nrhs
-        work = PRODUCTS[form] * flops
-        peak = PEAK["bf16_mfma"] if mixed else PEAK["fp64_mfma"]
-        kname, bound = ("k_m2l_mixed", "mfma") if mixed else ("k_m2l_f64", "mfma")
-        extra = {"m2l_interactions": n_int, "fp64_equivalent_flops_per_step": flops,
-                 "work": f"{PRODUCTS[form]} bf16 partial products per product" if mixed else "FP64 products"}
+        extra = {"m2l_interactions": n_int, "fp64_equivalent_flops_per_step": flops}
+        bound = "mfma"
+        if not mixed or engines[0].m2l_variant()[0] == F64_PRODUCTS:
+            work = sum(executed_m2l_flops(e, p) for e in engines) * nrhs
+            peak, kname = PEAK["fp64_mfma"], "k_m2l_up"
+            extra["work"] = "FP64 class products of k_m2l_up and k_m2l_down, 4 p^3 flops per cell and rank of the 56 offsets"
+        else:
+            work = PRODUCTS[form] * flops
+            peak, kname = PEAK["bf16_mfma"], "k_m2l_mixed"
+            extra["work"] = f"{PRODUCTS[form]} bf16 partial products per product"
     elif top in (p2p_small, p2p_big, "p2p_mixed_mutual"):
         pairs = {"small": 0.0, "big": 0.0, "big_big": 0.0, "big_rest": 0.0}
         for e in engines:
@@ -266,19 +293,18 @@ def roofline(engines, kernel_ms, launches, p, form, workload, nrhs=1, kernel=Non
                 pairs[k] += v * nrhs
         peak = PEAK["fp32_vector"] if mixed else PEAK["fp64_vector"]
         bound = "valu"
-        if top == "p2p_mixed_mutual":
+        if top in ("p2p_mixed_mutual", "p2p_big"):
             # each unordered big-big pair once (39 flops, the reference's mutual
             # count), the other pairs of the big leaves one way (34 flops)
             work = 39.0 * pairs["big_big"] / 2 + 34.0 * pairs["big_rest"]
-            kname = "k_p2p_mixed_mutual"
+            kname = "k_p2p_mixed_mutual" if mixed else "k_p2p_f64_mutual"
             extra = {"pairs": pairs["big"], "unordered_big_big_pairs": pairs["big_big"] / 2,
                      "ordered_other_pairs": pairs["big_rest"],
                      "work": "39 flops per unordered pair of two big leaves, 34 per other target-source pair "
                              "(FChebFlopsSymKernel.hpp:66-69)"}
         else:
             work = 34.0 * (pairs["big"] if top == p2p_big else pairs["small"])
-            kname = {"p2p_mixed": "k_p2p_mixed", "p2p_mixed_big": "k_p2p_mixed_big", "p2p": "k_p2p_f64",
-                     "p2p_big": "k_p2p_f64_big"}[top]
+            kname = {"p2p_mixed": "k_p2p_mixed", "p2p_mixed_big": "k_p2p_mixed_big", "p2p": "k_p2p_f64"}[top]
             extra = {"pairs": pairs["big"] if top == p2p_big else pairs["small"],
                      "work": "34 flops per target-source pair"}
     else:
@@ -555,7 +581,7 @@ def main():
         "metric": METRIC, "value": value, "unit": "Mparticles/s", "n_gpus": 1, "steps": args.steps,
         "warmup": args.warmup, "ms_per_step": ms, "higher_is_better": True, "scaling": "weak",
         "vs_baseline": None,
-        "dtype": DTYPE[args.precision],
+        "dtype": dtype_of(args.precision, m2l_variant[0]),
         "data": "synthetic",
         "config": {"workload": args.workload, "particles": n, "distribution": dist,
                    "seed": SEED[dist], "height": h, "order": p, "epsilon": 10.0 ** -p, "precision": args.precision},

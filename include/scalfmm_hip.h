@@ -55,7 +55,8 @@ extern "C" {
 /* ---- precision modes ------------------------------------------------------ */
 #define HFMM_PRECISION_FP64 0 /* every kernel in FP64 (the reference's FReal=double) */
 #define HFMM_PRECISION_MIXED 1 /* M2L on bfloat16 matrix cores with three-part operand
-                                  splits and FP32 accumulation, P2P in FP32 with
+                                  splits and FP32 accumulation, or in FP64 where that
+                                  is faster (hfmm_set_m2l_variant), P2P in FP32 with
                                   compensated sums; P2M/M2M/L2L/L2P and all results in
                                   FP64.  Relative error about 1e-7 on top of the
                                   FP64 path's; no counterpart in the reference (its
@@ -405,11 +406,12 @@ int hfmm_operator_file_name(int32_t order, double epsilon, char* buf, int32_t si
 /* The mixed-precision M2L has several tile shapes: 0 = four waves share 64
  * targets (every order), 1 = one 16-target tile per wave (orders 5 and 6),
  * 2 = two 16-target tiles per wave (order 5), 3 = four waves share 32
- * targets (every order).  Variant -1 (the default) times
- * every available variant once at the next M2L on the actual tree and keeps
- * the fastest for the context's later evaluations.  The FP64 form has one
+ * targets (every order), and 4 = the FP64 form's products (orders 6 to 8, no
+ * bfloat16 rounding).  Variant -1 (the default) is 4 from order 6; at order 5 it
+ * times every available tile shape once at the next M2L on the actual tree and
+ * keeps the fastest for the context's later evaluations.  The FP64 form has one
  * kernel (its variant stays -1).  hfmm_get_m2l_variant also returns the
- * times (ms) the last tuning measured per variant (4 floats, 0 = not run).
+ * times (ms) the last tuning measured per tile shape (4 floats, 0 = not run).
  * No counterpart in the reference (its M2L has one CPU implementation). */
 int hfmm_set_m2l_variant(hfmm_ctx* ctx, int32_t variant);
 int hfmm_get_m2l_variant(hfmm_ctx* ctx, int32_t* variant, float* tune_ms);

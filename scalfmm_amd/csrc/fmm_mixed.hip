@@ -910,6 +910,7 @@ int m2l_mixed_wave_launch(Context* c) {
 //   2  two 16-target tiles per wave (p = 5)
 //   3  four waves share 32 targets (every order): half the registers and LDS
 //      of shape 0 for twice its operator reads per target
+//   4  the FP64 form's products (m2l_f64.hip), from order kF64ProductsOrder
 template <int P, int NPL>
 int m2l_mixed_variant(Context* c, int v) {
     switch (v) {
@@ -926,9 +927,17 @@ int m2l_mixed_variant(Context* c, int v) {
     return fail(c, HFMM_ERR_ARG, "mixed M2L variant not available at this order");
 }
 
-constexpr int kMixedVariants = 4;
+constexpr int kMixedVariants = 4;  // shapes that the autotuner times
+// The FP64 products share work between the positions that differ in signs and
+// pad ranks to 4: from this order they beat every bfloat16 shape, without its
+// rounding, so that a context whose variant is not set takes them.  M2L with its
+// conversions, best shape of three / two parts against FP64, in ms: 1M uniform
+// h7 order 6 19.0 / 13.7, 8.5, order 7 31.3 / 24.6, 16.1, order 8 43.1 / 33.8, 25.1;
+// 30k uniform h5 order 6 0.62 / 0.64, 0.23; 1.25M Plummer h7 order 8 12.0 / 8.7,
+// 6.1; 10M Plummer h8 order 8 78 / 60.6, 57.8.
+constexpr int kF64Products = 4, kF64ProductsOrder = 6;
 inline bool mixed_variant_ok(int p, int v) {
-    return v == 0 || v == 3 || (v == 1 && p <= kWaveM2LMaxOrder) || (v == 2 && p <= 5);
+    return (v == kF64Products && p >= kF64ProductsOrder) || v == 0 || v == 3 || (v == 1 && p <= kWaveM2LMaxOrder) || (v == 2 && p <= 5);
 }
 
 // Times every available variant once on the current tree (each writes every
@@ -1056,6 +1065,7 @@ int run_split_multipoles(Context* c) {
 
 int run_m2l_mixed(Context* c) {
     if (c->kpad_max > 64) return fail(c, HFMM_ERR_ARG, "operator rank above 64 is not supported");
+    HFMM_TRY(ensure_parity_order(c));
     // three-part splits (six products) or, in HFMM_PRECISION_MIXED_HILO, two-part
     // hi/lo splits (three products)
     const bool hilo = c->P.precision == HFMM_PRECISION_MIXED_HILO;
@@ -1071,7 +1081,15 @@ int run_m2l_mixed(Context* c) {
 int m2l_variant_count(Context* c) { return is_mixed(c) ? kMixedVariants : 1; }
 bool m2l_variant_available(Context* c, int v) {
     if (!is_mixed(c)) return v == 0;
-    return v >= 0 && v < kMixedVariants && mixed_variant_ok(c->order(), v);
+    return v >= 0 && mixed_variant_ok(c->order(), v);
+}
+
+int m2l_takes_f64(Context* c, bool& f64) {
+    f64 = !is_mixed(c);
+    if (f64) return HFMM_OK;
+    if (c->m2l_variant < 0 && c->order() >= kF64ProductsOrder) c->m2l_variant = kF64Products;
+    f64 = c->m2l_variant == kF64Products;
+    return f64 && c->m2l_nrb == 0 ? prepare_m2l_f64(c) : HFMM_OK;
 }
 
 int selftest_mfma_bf16(Context* c, float* out) {

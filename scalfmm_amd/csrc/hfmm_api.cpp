@@ -195,6 +195,7 @@ static int upload_operators(Context* c) {
     HFMM_HIP(c, hipMemcpy(c->d_slotord.ptr, so.data(), sizeof(int16_t) * so.size(), hipMemcpyHostToDevice));
     HFMM_TRY(ensure(c, c->d_slotseg, sizeof(int32_t) * seg.size()));
     HFMM_HIP(c, hipMemcpy(c->d_slotseg.ptr, seg.data(), sizeof(int32_t) * seg.size(), hipMemcpyHostToDevice));
+    c->m2l_nrb = 0;
     return is_mixed(c) ? HFMM_OK : prepare_m2l_f64(c);
 }
 
@@ -213,7 +214,7 @@ static void free_all(Context* c) {
                       &c->d_count, &c->d_cellkey, &c->d_childstart, &c->d_leafstart,
                       &c->d_p2p, &c->d_p2pitems, &c->d_m2l, &c->d_order, &c->d_pcount, &c->d_dense, &c->d_M, &c->d_L, &c->d_Mb, &c->d_loc, &c->d_res_sorted, &c->d_qall,
                       &c->d_res, &c->d_field, &c->d_setoff, &c->d_keep, &c->d_kept, &c->d_gBt, &c->d_gU, &c->d_gC, &c->d_gCr, &c->d_Mt, &c->d_Lt, &c->d_uroots, &c->d_uK, &c->d_utw,
-                      &c->d_m2lrows, &c->d_m2ltab, &c->d_m2lup, &c->d_m2ldown, &c->d_m2lC, &c->d_m2lacc, &c->d_p2pitems_m, &c->d_itemkeys, &c->d_itemidx, &c->d_items_tmp, &c->d_direct, &c->d_csoff, &c->d_csparts, &c->d_csbase, &c->d_cpart};
+                      &c->d_m2lops, &c->d_m2lC, &c->d_m2lacc, &c->d_p2pitems_m, &c->d_itemkeys, &c->d_itemidx, &c->d_items_tmp, &c->d_direct, &c->d_csoff, &c->d_csparts, &c->d_csbase, &c->d_cpart};
     for (DevBuf* b : bufs) release(*b);
 }
 
@@ -391,7 +392,9 @@ static int evaluate_passes(Context* c, uint32_t ops, size_t exp_bytes) {
     } else if (ops & HFMM_M2L) {
         HFMM_TRY(accumulating(c, Lx, static_cast<int64_t>(exp_bytes / sizeof(double)), [&] {
             if (keep || !all_levels) HFMM_TRY(hfmm::zero_device(c, c->d_L.ptr, exp_bytes));
-            if (!mixed) return hfmm::run_m2l(c);
+            bool f64 = false;
+            HFMM_TRY(hfmm::m2l_takes_f64(c, f64));
+            if (f64) return hfmm::run_m2l(c);
             HFMM_TRY(hfmm::run_split_multipoles(c));
             return hfmm::run_m2l_mixed(c);
         }));

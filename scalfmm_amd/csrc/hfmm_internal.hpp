@@ -94,8 +94,10 @@ struct Context {
     // FP64 M2L (m2l_f64.hip): rows of all offsets, tables, operator fragments of
     // the two products, the compressed expansions between them, and the partial
     // locals of a launch over parts of the rows
-    DevBuf d_m2lrows, d_m2ltab, d_m2lup, d_m2ldown, d_m2lC, d_m2lacc;
-    int m2l_nrb = 0;             // row blocks of 16
+    DevBuf d_m2lops, d_m2lC, d_m2lacc;
+    double *m2l_up = nullptr, *m2l_down = nullptr;  // the fragments in d_m2lops
+    size_t m2l_slots_at = 0;                        // the slot table in d_m2lops
+    int m2l_nrb = 0;             // row blocks of 16 (0: not prepared)
     std::vector<int> m2l_rboff;  // bytes of a target's C before each row block
     int m2l_variant = -1;    // M2L kernel variant; -1: pick by timing at the next M2L
     float m2l_tune_ms[4] = {0.f, 0.f, 0.f, 0.f};  // times measured by the last autotune
@@ -343,6 +345,9 @@ int run_m2l_mixed(Context* c);
 int run_p2p_mixed(Context* c);
 int m2l_variant_count(Context* c);
 bool m2l_variant_available(Context* c, int v);
+// Whether this evaluation's M2L runs the FP64 products (the FP64 form, and the
+// mixed forms' variant 4, prepared on its first use).
+int m2l_takes_f64(Context* c, bool& f64);
 int selftest_mfma_bf16(Context* c, float* out);
 
 // FP64 direct sum for sampled targets (direct.hip)

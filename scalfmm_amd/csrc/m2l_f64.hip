@@ -32,6 +32,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <vector>
 
 #include "fmm_common.hpp"
@@ -786,18 +787,23 @@ __global__ __launch_bounds__(256) void k_m2l_pack(const RowInfo* __restrict__ ro
     }
 }
 
+// The tables and fragments in one device buffer: `tables` (rows, offsets, slot
+// table), then the fragments of the upward and of the downward product.
 template <int P>
-int pack_impl(Context* c, int nrb, const TauInfo* tau) {
+int pack_impl(Context* c, int nrb, const std::vector<char>& tables, size_t tau_at) {
     using K = Cls<P>;
-    HFMM_TRY(ensure(c, c->d_m2lup, sizeof(double) * static_cast<size_t>(nrb) * K::up_off(8)));
-    HFMM_TRY(ensure(c, c->d_m2ldown, sizeof(double) * static_cast<size_t>(nrb) * K::down_off(8)));
-    hipLaunchKernelGGL(k_m2l_pack<P>, dim3(nrb, kMWaves, 2), dim3(256), 0, c->stream, c->d_m2lrows.as<RowInfo>(), tau,
+    const size_t up_at = (tables.size() + 255) & ~size_t(255);
+    const size_t up = static_cast<size_t>(nrb) * K::up_off(8), down = static_cast<size_t>(nrb) * K::down_off(8);
+    HFMM_TRY(ensure(c, c->d_m2lops, up_at + sizeof(double) * (up + down)));
+    char* base = c->d_m2lops.as<char>();
+    c->m2l_up = reinterpret_cast<double*>(base + up_at);
+    c->m2l_down = c->m2l_up + up;
+    HFMM_HIP(c, hipMemcpy(base, tables.data(), tables.size(), hipMemcpyHostToDevice));
+    hipLaunchKernelGGL(k_m2l_pack<P>, dim3(nrb, kMWaves, 2), dim3(256), 0, c->stream,
+                       reinterpret_cast<const RowInfo*>(base), reinterpret_cast<const TauInfo*>(base + tau_at),
                        c->d_pidx.as<uint32_t>(), c->d_pvec.as<uint16_t>(), c->d_rank.as<int32_t>(),
-                       c->d_opoff.as<int64_t>(), c->d_ops.as<double>(), c->LD, c->d_m2lup.as<double>(),
-                       c->d_m2ldown.as<double>());
-    HFMM_TRY(check_launch(c, "m2l_pack"));
-    HFMM_HIP(c, hipStreamSynchronize(c->stream));
-    return HFMM_OK;
+                       c->d_opoff.as<int64_t>(), c->d_ops.as<double>(), c->LD, c->m2l_up, c->m2l_down);
+    return check_launch(c, "m2l_pack");
 }
 
 // Device memory for C: what a buffer reaches.  Larger trees run the rows in
@@ -847,14 +853,14 @@ int m2l_launch(Context* c, M2LArgs a) {
         a.stride = c->m2l_rboff[cut[i + 1]] - a.off0;
         a.load = i > 0;
         a.store = i + 1 < parts;
-        a.ops = c->d_m2lup.as<double>();
-        prof_begin(c, "m2l");
+        a.ops = c->m2l_up;
+        prof_begin(c, is_mixed(c) ? "m2l_mixed" : "m2l");
         hipLaunchKernelGGL((k_m2l_up<P, C, WIDE>), dim3(static_cast<unsigned>(grid)), dim3(kMThreads), su.bytes, c->stream, a,
                            su, c->d_M.as<double>(), c->LD);
         prof_end(c);
         HFMM_TRY(check_launch(c, "m2l_up"));
-        a.ops = c->d_m2ldown.as<double>();
-        prof_begin(c, "m2l");
+        a.ops = c->m2l_down;
+        prof_begin(c, is_mixed(c) ? "m2l_mixed" : "m2l");
         hipLaunchKernelGGL((k_m2l_down<P, C>), dim3(static_cast<unsigned>(grid)), dim3(kMThreads), sd.bytes, c->stream,
                            a, sd, c->d_L.as<double>(), c->LD);
         prof_end(c);
@@ -875,8 +881,8 @@ int m2l_impl(Context* c) {
     if (a.ncell <= 0) return HFMM_OK;
     a.slots = c->d_m2l.as<int32_t>();
     a.keys = c->d_cellkey.as<uint64_t>();
-    a.rows = c->d_m2lrows.as<RowInfo>();
-    a.slot_tau = c->d_m2ltab.as<uint16_t>();
+    a.rows = c->d_m2lops.as<RowInfo>();
+    a.slot_tau = reinterpret_cast<const uint16_t*>(c->d_m2lops.as<char>() + c->m2l_slots_at);
     int step = 0;
     for (int b = 0; b < c->m2l_nrb; ++b) step = std::max(step, c->m2l_rboff[b + 1] - c->m2l_rboff[b]);
     if (static_cast<size_t>(step) * a.ncell > kBufferMax) return m2l_launch<P, 2, true>(c, a);
@@ -963,14 +969,15 @@ int prepare_m2l_f64(Context* c) {
     }
     c->m2l_rboff[nrb] = off;
     c->m2l_nrb = nrb;
-    const size_t rbytes = sizeof(RowInfo) * rows.size();
-    HFMM_TRY(ensure(c, c->d_m2lrows, rbytes + sizeof(tau)));
-    HFMM_HIP(c, hipMemcpy(c->d_m2lrows.ptr, rows.data(), rbytes, hipMemcpyHostToDevice));
-    TauInfo* dtau = reinterpret_cast<TauInfo*>(c->d_m2lrows.as<char>() + rbytes);
-    HFMM_HIP(c, hipMemcpy(dtau, tau, sizeof(tau), hipMemcpyHostToDevice));
-    HFMM_TRY(ensure(c, c->d_m2ltab, sizeof(uint16_t) * slot_tau.size()));
-    HFMM_HIP(c, hipMemcpy(c->d_m2ltab.ptr, slot_tau.data(), sizeof(uint16_t) * slot_tau.size(), hipMemcpyHostToDevice));
-#define CALL(P) pack_impl<P>(c, nrb, dtau)
+    const size_t tau_at = sizeof(RowInfo) * rows.size();
+    c->m2l_slots_at = tau_at + sizeof(tau);
+    std::vector<char> tables(c->m2l_slots_at + sizeof(uint16_t) * slot_tau.size());
+    std::memcpy(tables.data(), rows.data(), tau_at);
+    std::memcpy(tables.data() + tau_at, tau, sizeof(tau));
+    std::memcpy(tables.data() + c->m2l_slots_at, slot_tau.data(), sizeof(uint16_t) * slot_tau.size());
+    // an earlier evaluation may still read the old tables
+    HFMM_HIP(c, hipStreamSynchronize(c->stream));
+#define CALL(P) pack_impl<P>(c, nrb, tables, tau_at)
     HFMM_DISPATCH(c->order(), CALL)
 #undef CALL
 }

@@ -1022,11 +1022,11 @@ int build_tree_device(Context* c) {
     c->p2p_mutual = false;
     c->order_built = false;
     if (c->p2p_items_cap > 0) HFMM_TRY(build_p2p_mutual_tables(c, nbig));
-    return is_mixed(c) ? ensure_parity_order(c) : HFMM_OK;
+    return HFMM_OK;
 }
 
-// The cells of every level by child index (mixed and global-SVD M2L; the
-// symmetric FP64 M2L takes them as they are).
+// The cells of every level by child index, for the M2L kernels that read them so
+// (bfloat16 tiles, global SVD), once per tree.
 int ensure_parity_order(Context* c) {
     if (c->order_built) return HFMM_OK;
     ParityLevels lv{};

@@ -311,7 +311,7 @@ class Engine:
         return off, sr[:m], ps[:m]
 
     def set_m2l_variant(self, v):
-        """Mixed M2L tile shape (0, 1, 2, 3) or -1 to autotune at the next M2L."""
+        """Mixed M2L tile shape (0 to 3), 4 for the FP64 products (orders 6 to 8), or -1 to choose at the next M2L."""
         self._check(self._L.hfmm_set_m2l_variant(self.h, int(v)))
 
     def m2l_variant(self):

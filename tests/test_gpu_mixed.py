@@ -253,3 +253,31 @@ def test_hilo_plummer_order5_vs_direct(oracle, plummer100k):
         e.close()
     _say(f"  pot rel L2 vs direct: fp64 {errs['fp64']:.3e} hilo {errs['hilo']:.3e}")
     assert errs["hilo"] <= 1.01 * errs["fp64"]
+
+
+@pytest.mark.parametrize("order,h,n,hilo", [(6, 5, 20000, False), (7, 4, 3000, True), (8, 4, 3001, False)])
+def test_mixed_f64_products(oracle, order, h, n, hilo):
+    """A context whose variant is not set takes the FP64 form's M2L from order 6:
+    the far field within the FP64 path's 1e-12 of the oracle, the same bits
+    when the variant is set, and the bfloat16 tiles still there."""
+    from scalfmm_amd import PRECISION_MIXED, PRECISION_MIXED_HILO, Engine, FFmmFarField
+    from scalfmm_amd.distributions import uniform_cube
+    x, y, z, q = uniform_cube(n, 31)
+    ref = oracle.fmm(x, y, z, q, (0.5, 0.5, 0.5), 1.0, h, order, ops=FFmmFarField)
+    got = {}
+    for v in (None, 4, 0):
+        e = Engine(h, 1.0, (0.5, 0.5, 0.5), order, 0.0, 0, PRECISION_MIXED_HILO if hilo else PRECISION_MIXED)
+        if v is not None:
+            e.set_m2l_variant(v)
+        e.set_particles(x, y, z, q)
+        e.build_tree()
+        e.evaluate(FFmmFarField)
+        assert e.m2l_variant()[0] == (4 if v is None else v)
+        got[v] = e.results()
+        e.close()
+    for a, b, c, r in zip(got[None], got[4], got[0], ref[:4]):
+        assert np.array_equal(a, b)
+        assert _rel(a, r) <= 1e-12
+        assert _rel(c, r) <= (6e-5 if hilo else 3e-6)
+    with pytest.raises(Exception):
+        Engine(4, 1.0, (0.5, 0.5, 0.5), 5, 0.0, 0, PRECISION_MIXED).set_m2l_variant(4)
