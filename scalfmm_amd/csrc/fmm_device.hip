@@ -566,8 +566,7 @@ __global__ __launch_bounds__(256) void k_p2p_f64_rhs(int64_t n, const int32_t* _
 // wave-uniform, so the sources arrive through scalar loads into SGPRs and
 // feed the FP64 arithmetic as scalar operands (no LDS, no barriers).  A block
 // running past the leaf's end masks the extra sources (the sorted arrays are
-// padded, so the reads stay in bounds).  Sources are summed in the same order
-// as k_p2p_f64.
+// padded with zeros, so the reads stay in bounds and find numbers).
 constexpr int kP2PBlock64 = 8;
 
 template <bool MASK>

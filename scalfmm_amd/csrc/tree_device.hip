@@ -340,6 +340,9 @@ __global__ __launch_bounds__(kBlock) void k_gather_particles(int64_t n, const in
                                                             double* __restrict__ out, int32_t* __restrict__ iperm) {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= n) return;
+    // the padding that masked sources read: their charge has to be a number
+    if (i == 0)
+        for (int k = 0; k < kSortedPad; ++k) out[4 * n + k] = 0.;
     const int32_t o = idx[i];
     iperm[o] = static_cast<int32_t>(i);
     out[i] = x[o];

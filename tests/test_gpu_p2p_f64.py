@@ -44,3 +44,32 @@ def test_f64_mutual_p2p(oracle, ops):
         e.close()
     for a, b in zip(out[True], out[False]):
         assert _rel(a, b) <= 1e-12
+
+
+def test_last_leaf_reads_clean_padding(oracle):
+    """The masked sources past a big last leaf read the padding of the sorted
+    arrays: finite results also where that memory held NaN before."""
+    from scalfmm_amd import Engine, FFmmNearField
+    rng = np.random.default_rng(6)
+    n = 1021
+    x, y, z = 0.75 + 0.24 * rng.random((3, n))  # one leaf
+    q = 2.0 * rng.random(n) - 1.0
+    ref = oracle.fmm(x, y, z, q, (0.5, 0.5, 0.5), 1.0, H, 5, ops=FFmmNearField)
+    for mutual in (True, False):
+        for charges in (np.full(n, np.nan), q):
+            e = Engine(H, 1.0, (0.5, 0.5, 0.5), 5)
+            e.set_p2p_mutual(mutual)
+            # the arrays of 4 more particles hold NaN where the next ones have their padding
+            extra = 4 if np.isnan(charges[0]) else 0
+            e.set_particles(*(np.concatenate([a, a[:extra]]) for a in (x, y, z)), np.concatenate([charges, charges[:extra]]))
+            e.build_tree()
+            e.evaluate(FFmmNearField)
+            got = e.results()
+            if extra:  # the same context again, on the buffers it has
+                e.set_particles(x, y, z, q)
+                e.build_tree()
+                e.evaluate(FFmmNearField)
+                got = e.results()
+            e.close()
+            for a, b in zip(got, ref[:4]):
+                assert _rel(a, b) <= 1e-12
