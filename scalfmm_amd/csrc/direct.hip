@@ -87,9 +87,17 @@ __global__ __launch_bounds__(kDirectBlock) void k_direct_sum(const double* __res
                                                             const double* __restrict__ part, double* __restrict__ out) {
     const int64_t g = static_cast<int64_t>(blockIdx.x) * kDirectBlock + threadIdx.x;
     if (g >= nt) return;
-    double s[4] = {0., 0., 0., 0.};
+    // compensated (each addition's exact error is carried along): dozens of plain
+    // additions cost the last digit of sums whose terms have one sign
+    double s[4] = {0., 0., 0., 0.}, e[4] = {0., 0., 0., 0.};
     for (int i = 0; i < shares; ++i)
-        for (int k = 0; k < 4; ++k) s[k] += part[(static_cast<int64_t>(i) * 4 + k) * nt + g];
+        for (int k = 0; k < 4; ++k) {
+            const double v = part[(static_cast<int64_t>(i) * 4 + k) * nt + g], t = s[k] + v, w = t - s[k];
+            e[k] += (s[k] - (t - w)) + (v - w);
+            s[k] = t;
+        }
+    // a sum that left the finite numbers stands as it is
+    for (int k = 0; k < 4; ++k) s[k] = isfinite(s[k]) ? s[k] + e[k] : s[k];
     const double qt = q[targets[g]];
     out[g] = s[0];
     for (int k = 1; k < 4; ++k) out[k * nt + g] = s[k] * qt;
