@@ -934,7 +934,7 @@ constexpr int kMixedVariants = 4;  // shapes that the autotuner times
 // conversions, best shape of three / two parts against FP64, in ms: 1M uniform
 // h7 order 6 19.0 / 13.7, 8.5, order 7 31.3 / 24.6, 16.1, order 8 43.1 / 33.8, 25.1;
 // 30k uniform h5 order 6 0.62 / 0.64, 0.23; 1.25M Plummer h7 order 8 12.0 / 8.7,
-// 6.1; 10M Plummer h8 order 8 78 / 60.6, 57.8.
+// 6.1; 10M Plummer h8 order 8 78 / 60.6, 42.0.
 constexpr int kF64Products = 4, kF64ProductsOrder = 6;
 inline bool mixed_variant_ok(int p, int v) {
     return (v == kF64Products && p >= kF64ProductsOrder) || v == 0 || v == 3 || (v == 1 && p <= kWaveM2LMaxOrder) || (v == 2 && p <= 5);

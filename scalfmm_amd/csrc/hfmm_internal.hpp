@@ -97,6 +97,8 @@ struct Context {
     DevBuf d_m2lops, d_m2lC, d_m2lacc;
     double *m2l_up = nullptr, *m2l_down = nullptr;  // the fragments in d_m2lops
     size_t m2l_slots_at = 0;                        // the slot table in d_m2lops
+    size_t m2l_room = 0;         // bytes that C may take, where a buffer's reach is too little
+    bool m2l_short = false;      // the device had no room for more
     int m2l_nrb = 0;             // row blocks of 16 (0: not prepared)
     std::vector<int> m2l_rboff;  // bytes of a target's C before each row block
     int m2l_variant = -1;    // M2L kernel variant; -1: pick by timing at the next M2L

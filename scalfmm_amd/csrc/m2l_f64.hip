@@ -28,6 +28,12 @@
 // classes are dealt to give every SIMD the same number of MFMAs (order 7: 23,
 // 21, 21, 21 per 16 rows).  A step is 32 (row, cell) lines of 16; the tile that
 // holds the Hadamard operands is double buffered, one barrier per step.
+//
+// Bound by the SIMDs: MFMAs 45-50% of the time, and FP64 MFMAs and VALU
+// instructions do not overlap (4 VALU instructions beside a 66-cycle MFMA add 16
+// cycles); the rest is the transform's VALU work and waits at the barriers.  1M
+// uniform particles, h7, order 7: 55.7 (one operator per slot) -> 15.8 ms, 33.9
+// TFLOP/s executed; 10M Plummer, h8, order 8: 202 -> 42 ms.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -806,15 +812,42 @@ int pack_impl(Context* c, int nrb, const std::vector<char>& tables, size_t tau_a
     return check_launch(c, "m2l_pack");
 }
 
-// Device memory for C: what a buffer reaches.  Larger trees run the rows in
-// parts, whose partial locals pass through memory (p^3 doubles per cell and
-// part).  Where one step's C is larger still (more than 4 million cells),
-// addresses take 64 bits.
+// Device memory for C: all of it, or what kRoomMax and a quarter of the free
+// memory leave.  Beyond that the rows run in parts, each with the prologue of
+// every tile and with partial locals through memory (p^3 doubles per cell and
+// part).  Within a buffer's reach (4 GB) the upward kernel stores through a
+// buffer; beyond it with 64-bit addresses under a mask, which costs less than
+// the parts: 1M uniform h7, order 7 (12 GB) 17.2 ms in three parts, 16.4 in
+// one; 192 sets x 8 vectors, order 5, 51.0 / 48.5; 12M uniform h9, order 5, a
+// pass of 2,783 ms one step at a time, 730 with 32 GB, 530 with 64.
 constexpr int kMaxPart = 116;  // row blocks of a launch: their table fits the LDS beside the tiles
-constexpr int64_t kTwoTiles = 16 * 1024;  // cells from which a workgroup takes two column tiles
+constexpr size_t kRoomMax = size_t(32) << 30;
+
+// Bytes that C may take of `want` (more than a buffer's reach).  The device is
+// asked only where a context wants more than before and got all of that, so that
+// a captured run decides as the run before it.
+size_t room_for_c(Context* c, size_t want) {
+    if (want > c->m2l_room && !c->m2l_short) {
+        size_t free_b = 0, total_b = 0;
+        if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) (void)hipGetLastError();
+        c->m2l_room = std::max(c->m2l_room, std::min(want, (free_b + c->d_m2lC.bytes) / 4));
+        c->m2l_short = c->m2l_room < want;
+    }
+    return std::min(want, c->m2l_room);
+}
+
+// Two column tiles per workgroup (32 cells) reuse the operators but take 1.7
+// times as long as one (1,000 uniform particles, order 7: 354 against 205 us), so
+// they pay where they need fewer rounds of the 256 CUs: 585 cells, order 8, 575
+// against 338 us; 4,681 cells, order 5 139 / 154, order 8 595 / 711; 37,449 cells,
+// order 6 1,239 / 1,400.
+inline bool two_tiles(int64_t ncell) {
+    const int64_t one = (ncell + 16 * 256 - 1) / (16 * 256), two = (ncell + 32 * 256 - 1) / (32 * 256);
+    return 17 * two < 10 * one;
+}
 
 template <int P, int C, bool WIDE>
-int m2l_launch(Context* c, M2LArgs a) {
+int m2l_launch(Context* c, M2LArgs a, size_t room) {
     using K = Cls<P>;
     constexpr int RB = Lds<C>::RB;
     const int nrb = c->m2l_nrb;
@@ -827,7 +860,7 @@ int m2l_launch(Context* c, M2LArgs a) {
         int e = cut.back() + RB;
         auto width = [&](int to) { return c->m2l_rboff[to] - c->m2l_rboff[cut.back()]; };
         while (e < nrb && e + RB - cut.back() <= kMaxPart &&
-               static_cast<size_t>(width(std::min(e + RB, nrb))) * a.ncell <= kBufferMax) e += RB;
+               static_cast<size_t>(width(std::min(e + RB, nrb))) * a.ncell <= room) e += RB;
         e = std::min(e, nrb);
         stride = std::max<int64_t>(stride, width(e));
         cut.push_back(e);
@@ -885,8 +918,11 @@ int m2l_impl(Context* c) {
     a.slot_tau = reinterpret_cast<const uint16_t*>(c->d_m2lops.as<char>() + c->m2l_slots_at);
     int step = 0;
     for (int b = 0; b < c->m2l_nrb; ++b) step = std::max(step, c->m2l_rboff[b + 1] - c->m2l_rboff[b]);
-    if (static_cast<size_t>(step) * a.ncell > kBufferMax) return m2l_launch<P, 2, true>(c, a);
-    return a.ncell >= kTwoTiles ? m2l_launch<P, 2, false>(c, a) : m2l_launch<P, 1, false>(c, a);
+    const size_t all = std::min(static_cast<size_t>(c->m2l_rboff[c->m2l_nrb]) * a.ncell, kRoomMax);
+    const size_t room = all > kBufferMax ? room_for_c(c, all) : 0;
+    if (room > kBufferMax) return m2l_launch<P, 2, true>(c, a, room);
+    if (static_cast<size_t>(step) * a.ncell > kBufferMax) return m2l_launch<P, 2, true>(c, a, kBufferMax);
+    return two_tiles(a.ncell) ? m2l_launch<P, 2, false>(c, a, kBufferMax) : m2l_launch<P, 1, false>(c, a, kBufferMax);
 }
 
 #define HFMM_DISPATCH(P_, CALL)                                                   \

@@ -1,5 +1,5 @@
 """The FP64 M2L at the edges of its tiles against the oracle: fewer cells than a
-column tile, partly filled tiles, both tile shapes (below and above 16,384
+column tile, partly filled tiles, both tile shapes (by the number of
 cells), every order, and sparse trees whose tiles skip offsets.  Locals and
 results to 1e-12 relative L2, the bound of the FP64 path."""
 import numpy as np
@@ -19,7 +19,7 @@ CASES = [
     (uniform_cube, 3001, 4, 8),
     (plummer, 20011, 6, 5),  # sparse: tiles without some of the offsets
     (plummer, 20011, 7, 7),
-    (uniform_cube, 45001, 6, 5),  # above 16,384 cells: two column tiles per workgroup
+    (uniform_cube, 45001, 6, 5),  # 18,000 cells and more: two column tiles per workgroup
     (uniform_cube, 45001, 6, 6),
     (uniform_cube, 45001, 6, 7),
     (uniform_cube, 45001, 6, 8),
@@ -64,3 +64,25 @@ def test_m2l_tile_shapes_agree():
             for g, r in zip(got, e.results()):
                 assert np.array_equal(g[a:b], r)
         e.close()
+
+
+@pytest.mark.parametrize("p", [7, 8])
+def test_m2l_wide_addresses_agree(p):
+    """Compressed expansions within 4 GB (each set alone) and beyond (64-bit
+    addresses): the same bits."""
+    x, y, z, q = uniform_cube(130003, 29)
+    off = [0, 35001, 75002, 130003]
+    e = Engine(7, 1.0, CENTER, p)
+    e.set_particle_sets(off, x, y, z, q)
+    e.build_tree()
+    e.evaluate()
+    got = e.results()
+    a, b = off[0], off[1]
+    e.close()
+    e = Engine(7, 1.0, CENTER, p)
+    e.set_particles(x[a:b], y[a:b], z[a:b], q[a:b])
+    e.build_tree()
+    e.evaluate()
+    for g, r in zip(got, e.results()):
+        assert np.array_equal(g[a:b], r)
+    e.close()
