@@ -43,14 +43,13 @@
 
 #include "fmm_common.hpp"
 #include "hfmm_internal.hpp"
+#include "m2l_plan.hpp"
 
 namespace hfmm {
 namespace {
 
 typedef double d4 __attribute__((ext_vector_type(4)));
 
-constexpr int kTau = 56;       // offsets (|x|, |y|, |z|), far field
-constexpr int kTauDummy = 56;  // of the rows that fill the last row block
 constexpr int kTauStride = 60; // bytes per cell of a table over the offsets (whole words)
 constexpr int kMWaves = 8;
 constexpr int kMThreads = 64 * kMWaves;
@@ -110,14 +109,6 @@ struct Cls {
     }
 };
 
-// One row of the products: its offset |pos|, its place in a target's C (bytes,
-// variant 0), and the bytes that a negative sign of each coordinate adds (0:
-// only one sign, or none, belongs to the offset).
-struct __attribute__((aligned(16))) RowInfo {
-    uint32_t tau, off;
-    uint16_t sign[3], pad;
-};
-
 struct M2LArgs {
     M2LLevels lv;
     int64_t first, ncell;  // cells of the working levels
@@ -160,8 +151,6 @@ __device__ __forceinline__ void hadamard8(double (&d)[8]) {
 // store is dropped and a load gives 0, so a lane without a partner takes part
 // with the offset kNowhere.  A branch around each access would hide their number
 // from the wait counts: every wait for operators would wait for all stores.
-constexpr uint32_t kNowhere = 0xFFF00000u;  // plus an offset in a target's C (below 1 MiB)
-constexpr size_t kBufferMax = kNowhere;     // bytes
 
 typedef uint32_t u2 __attribute__((ext_vector_type(2)));
 
@@ -721,10 +710,6 @@ __global__ __launch_bounds__(kMThreads, 2) void k_m2l_down(M2LArgs a, SmemLayout
 // Operator fragments.  Entry of class k, half-node (hx, hy, hz), row (tau, r):
 // the mean over the mirror images of the node, with the class's signs, of
 // V_c[pv(|pos|)[n]][r] (up) or U_c (down).
-struct TauInfo {
-    int32_t pos, row0, rank, pad;
-};
-
 template <int P>
 __device__ double class_entry(const double* __restrict__ W, int kpad, const uint16_t* __restrict__ pv, int k, int m, int r) {
     using K = Cls<P>;
@@ -973,37 +958,8 @@ int prepare_m2l_f64(Context* c) {
             slot_tau[(8 + e) * kFarSlots + j] = static_cast<uint16_t>(8 * t + back);
         }
     }
-    // a target's C: row block by row block, in it per offset [variant][rows of
-    // the offset in the block]; a variant per pair of signs that a target of
-    // one parity has on an axis (|x| = 1, 2: both; 3: one, by its parity; 0: none)
-    std::vector<RowInfo> rows(static_cast<size_t>(nrb) * 16, RowInfo{kTauDummy, 0, {0, 0, 0}, 0});
-    for (int t = 0; t < kTau; ++t)
-        for (int r = 0; r < ((tau[t].rank + 3) & ~3); ++r) rows[tau[t].row0 + r].tau = static_cast<uint32_t>(t);
-    c->m2l_rboff.assign(nrb + 1, 0);
-    int off = 0;
-    for (int b = 0; b < nrb; ++b) {
-        c->m2l_rboff[b] = off;
-        for (int r = 0; r < 16;) {
-            const int t = static_cast<int>(rows[16 * b + r].tau);
-            int e = r;
-            while (e < 16 && static_cast<int>(rows[16 * b + e].tau) == t) ++e;
-            if (t != kTauDummy) {
-                const int v[3] = {tau[t].pos / 49 - 3, (tau[t].pos / 7) % 7 - 3, tau[t].pos % 7 - 3};
-                int bytes = 8 * (e - r);
-                uint16_t sign[3] = {0, 0, 0};
-                for (int a = 0; a < 3; ++a)
-                    if (v[a] == 1 || v[a] == 2) sign[a] = static_cast<uint16_t>(bytes), bytes *= 2;
-                for (int q = r; q < e; ++q) {
-                    RowInfo& ri = rows[16 * b + q];
-                    ri.off = static_cast<uint32_t>(off + 8 * (q - r));
-                    for (int a = 0; a < 3; ++a) ri.sign[a] = sign[a];
-                }
-                off += bytes;
-            }
-            r = e;
-        }
-    }
-    c->m2l_rboff[nrb] = off;
+    std::vector<RowInfo> rows;
+    row_layout(tau, nrb, rows, c->m2l_rboff);
     c->m2l_nrb = nrb;
     const size_t tau_at = sizeof(RowInfo) * rows.size();
     c->m2l_slots_at = tau_at + sizeof(tau);

@@ -1,0 +1,72 @@
+// m2l_plan.hpp -- host side of the FP64 M2L (m2l_f64.hip): the rows of the
+// products and their places in a target's compressed expansions C.
+#pragma once
+
+#include <cstddef>
+#include <cstdint>
+#include <vector>
+
+namespace hfmm {
+
+constexpr int kTau = 56;       // offsets (|x|, |y|, |z|), far field
+constexpr int kTauDummy = 56;  // of the rows that fill the last row block
+
+// Byte offset of a lane without a partner, past the end of every buffer, plus
+// the place of its row in a target's C (below 1 MiB, not negative).
+constexpr uint32_t kNowhere = 0xFFF00000u;
+constexpr size_t kBufferMax = kNowhere;  // bytes
+
+// One of the 56 offsets: its position in the 7^3 cube, first row and rank.
+struct TauInfo {
+    int32_t pos, row0, rank, pad;
+};
+
+// One row of the products: its offset |pos|, its place in a target's C (bytes,
+// variant 0), and the bytes that a negative sign of each coordinate adds (0:
+// only one sign, or none, belongs to the offset).
+struct __attribute__((aligned(16))) RowInfo {
+    uint32_t tau, off;
+    uint16_t sign[3], pad;
+};
+
+// A target's C: row block by row block, in it per offset [variant][rows of the
+// offset in the block]; a variant per pair of signs that a target of one parity
+// has on an axis (|x| = 1, 2: both; 3: one, by its parity; 0: none).  rboff:
+// bytes before each row block.  The rows that fill the last block lie at the end
+// of C, so that their place in a part of the rows (off minus the bytes before the
+// part) is not negative: added to kNowhere, off = 0 gave an address before
+// kNowhere, inside a buffer that reaches nearly that far.
+inline void row_layout(const TauInfo (&tau)[kTau], int nrb, std::vector<RowInfo>& rows, std::vector<int>& rboff) {
+    rows.assign(static_cast<size_t>(nrb) * 16, RowInfo{kTauDummy, 0, {0, 0, 0}, 0});
+    for (int t = 0; t < kTau; ++t)
+        for (int r = 0; r < ((tau[t].rank + 3) & ~3); ++r) rows[tau[t].row0 + r].tau = static_cast<uint32_t>(t);
+    rboff.assign(nrb + 1, 0);
+    int off = 0;
+    for (int b = 0; b < nrb; ++b) {
+        rboff[b] = off;
+        for (int r = 0; r < 16;) {
+            const int t = static_cast<int>(rows[16 * b + r].tau);
+            int e = r;
+            while (e < 16 && static_cast<int>(rows[16 * b + e].tau) == t) ++e;
+            if (t != kTauDummy) {
+                const int v[3] = {tau[t].pos / 49 - 3, (tau[t].pos / 7) % 7 - 3, tau[t].pos % 7 - 3};
+                int bytes = 8 * (e - r);
+                uint16_t sign[3] = {0, 0, 0};
+                for (int a = 0; a < 3; ++a)
+                    if (v[a] == 1 || v[a] == 2) sign[a] = static_cast<uint16_t>(bytes), bytes *= 2;
+                for (int q = r; q < e; ++q) {
+                    RowInfo& ri = rows[16 * b + q];
+                    ri.off = static_cast<uint32_t>(off + 8 * (q - r));
+                    for (int a = 0; a < 3; ++a) ri.sign[a] = sign[a];
+                }
+                off += bytes;
+            }
+            r = e;
+        }
+    }
+    rboff[nrb] = off;
+    for (RowInfo& ri : rows)
+        if (ri.tau == kTauDummy) ri.off = static_cast<uint32_t>(off);
+}
+
+}  // namespace hfmm

@@ -1,0 +1,32 @@
+"""csrc/m2l_plan.hpp through ctypes (a small library compiled by g++ on first use)."""
+import ctypes
+import functools
+import os
+import subprocess
+import tempfile
+
+import numpy as np
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+@functools.lru_cache(maxsize=None)
+def lib():
+    tmp = tempfile.TemporaryDirectory(prefix="m2l_plan")
+    out = os.path.join(tmp.name, "plan.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Wextra", "-Werror", "-shared", "-fPIC",
+                    os.path.join(HERE, "plan.cpp"), "-o", out], check=True)
+    L = ctypes.CDLL(out)
+    tmp.cleanup()  # the loaded library stays
+    L.plan_nowhere.restype = ctypes.c_uint32
+    return L
+
+
+def rows(rank):
+    """(offset index, place, largest place with signs) of every row and the bytes before each row block."""
+    rank = np.ascontiguousarray(rank, np.int32)
+    tau, off, last = (np.zeros(16 * 256, np.uint32) for _ in range(3))
+    rboff = np.zeros(257, np.int32)
+    nrb = lib().plan_rows(*(a.ctypes.data_as(ctypes.c_void_p) for a in (rank, tau, off, last, rboff)))
+    n = 16 * nrb
+    return tau[:n], off[:n], last[:n], rboff[: nrb + 1]
