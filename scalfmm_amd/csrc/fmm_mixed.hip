@@ -1085,10 +1085,8 @@ bool m2l_variant_available(Context* c, int v) {
 }
 
 int m2l_takes_f64(Context* c, bool& f64) {
-    f64 = !is_mixed(c);
-    if (f64) return HFMM_OK;
-    if (c->m2l_variant < 0 && c->order() >= kF64ProductsOrder) c->m2l_variant = kF64Products;
-    f64 = c->m2l_variant == kF64Products;
+    if (is_mixed(c) && c->m2l_variant < 0 && c->order() >= kF64ProductsOrder) c->m2l_variant = kF64Products;
+    f64 = !is_mixed(c) || c->m2l_variant == kF64Products;
     return f64 && c->m2l_nrb == 0 ? prepare_m2l_f64(c) : HFMM_OK;
 }
 

@@ -29,6 +29,7 @@ int ensure(Context* c, DevBuf& b, size_t bytes) {
     hipError_t e = hipMalloc(&b.ptr, bytes);
     if (e != hipSuccess) {
         b.ptr = nullptr;
+        (void)hipGetLastError();  // reported here, not by the next launch
         return fail(c, HFMM_ERR_NOMEM, std::string("hipMalloc(") + std::to_string(bytes) + "): " + hipGetErrorString(e));
     }
     b.bytes = bytes;

@@ -960,7 +960,6 @@ int prepare_m2l_f64(Context* c) {
     }
     std::vector<RowInfo> rows;
     row_layout(tau, nrb, rows, c->m2l_rboff);
-    c->m2l_nrb = nrb;
     const size_t tau_at = sizeof(RowInfo) * rows.size();
     c->m2l_slots_at = tau_at + sizeof(tau);
     std::vector<char> tables(c->m2l_slots_at + sizeof(uint16_t) * slot_tau.size());
@@ -969,9 +968,14 @@ int prepare_m2l_f64(Context* c) {
     std::memcpy(tables.data() + c->m2l_slots_at, slot_tau.data(), sizeof(uint16_t) * slot_tau.size());
     // an earlier evaluation may still read the old tables
     HFMM_HIP(c, hipStreamSynchronize(c->stream));
+    const auto pack = [&] {
 #define CALL(P) pack_impl<P>(c, nrb, tables, tau_at)
-    HFMM_DISPATCH(c->order(), CALL)
+        HFMM_DISPATCH(c->order(), CALL)
 #undef CALL
+    };
+    HFMM_TRY(pack());
+    c->m2l_nrb = nrb;  // prepared: not before the memory is there and the kernel on its way
+    return HFMM_OK;
 }
 
 int run_m2l(Context* c) {
