@@ -65,6 +65,19 @@ inline unsigned p2p_tiled_grid(const Context* c) {
     return static_cast<unsigned>(g > 0 ? g : 1);
 }
 
+// Workgroups of 256 threads for `threads` threads, in rows of at most 2^23: a
+// dimension of a launch holds fewer than 2^32 threads, and more are cut off
+// without an error.
+inline dim3 grid256(int64_t threads) {
+    constexpr int64_t kRow = int64_t(1) << 23;
+    const int64_t b = (threads + 255) / 256;
+    return b <= kRow ? dim3(static_cast<unsigned>(b)) : dim3(static_cast<unsigned>(kRow), static_cast<unsigned>((b + kRow - 1) / kRow));
+}
+// The thread's index in a launch over grid256.
+__device__ __forceinline__ int64_t thread_of_grid256() {
+    return (static_cast<int64_t>(blockIdx.y) * gridDim.x + blockIdx.x) * 256 + threadIdx.x;
+}
+
 // Raises a kernel's dynamic LDS limit to `bytes` when a launch needs more than
 // the default 64 KiB and more than set before on this device: the call is
 // made once per kernel and device, by an eager run, never while a stream is

@@ -542,7 +542,7 @@ __device__ __forceinline__ void p2p_f64_target(int64_t n, int64_t i, int g, cons
 __global__ __launch_bounds__(256) void k_p2p_f64(int64_t n, const int32_t* __restrict__ pleaf,
                                                 const int32_t* __restrict__ lstart, const int32_t* __restrict__ slots,
                                                 const double* __restrict__ sp, double* __restrict__ res) {
-    const int64_t i = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) / kP2PLanes;
+    const int64_t i = thread_of_grid256() / kP2PLanes;
     if (i >= n) return;
     p2p_f64_target<1>(n, i, threadIdx.x % kP2PLanes, pleaf, lstart, slots, sp, [&](int j, int) { return sp[3 * n + j]; }, res);
 }
@@ -554,7 +554,7 @@ __global__ __launch_bounds__(256) void k_p2p_f64_rhs(int64_t n, const int32_t* _
                                                     const int32_t* __restrict__ lstart,
                                                     const int32_t* __restrict__ slots, const double* __restrict__ sp,
                                                     const double* __restrict__ qc, double* __restrict__ res) {
-    const int64_t i = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) / kP2PLanes;
+    const int64_t i = thread_of_grid256() / kP2PLanes;
     if (i >= n) return;
     p2p_f64_target<R>(n, i, threadIdx.x % kP2PLanes, pleaf, lstart, slots, sp,
                       [&](int j, int r) { return qc[static_cast<int64_t>(j) * R + r]; }, res);
@@ -1035,7 +1035,7 @@ int run_l2p(Context* c) {
 int run_p2p(Context* c) {
     if (!c->p2p_small_done) {
         prof_begin(c, "p2p");
-        hipLaunchKernelGGL(k_p2p_f64, dim3(blocks256(c->n * kP2PLanes)), dim3(256), 0, c->stream, c->n, c->d_pleaf.as<int32_t>(),
+        hipLaunchKernelGGL(k_p2p_f64, grid256(c->n * kP2PLanes), dim3(256), 0, c->stream, c->n, c->d_pleaf.as<int32_t>(),
                            c->d_leafstart.as<int32_t>(), c->d_p2p.as<int32_t>(), c->d_sorted.as<double>(),
                            sorted_results(c));
         prof_end(c);
@@ -1109,7 +1109,7 @@ int run_p2p_small_all(Context* c) {
     for (int k = 0; k < nch; ++k) {
         const double* qc = c->d_qall.as<double>() + npad * ch[k].r0;
         double* res = c->d_res_sorted.as<double>() + static_cast<size_t>(ch[k].r0) * 4 * c->n;
-        const dim3 grid(blocks256(c->n * kP2PLanes)), block(256);
+        const dim3 grid = grid256(c->n * kP2PLanes), block(256);
         const int32_t* pl = c->d_pleaf.as<int32_t>();
         const int32_t* ls = c->d_leafstart.as<int32_t>();
         const int32_t* sl = c->d_p2p.as<int32_t>();
