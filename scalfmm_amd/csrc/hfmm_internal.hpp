@@ -97,8 +97,8 @@ struct Context {
     DevBuf d_m2lops, d_m2lC, d_m2lacc;
     double *m2l_up = nullptr, *m2l_down = nullptr;  // the fragments in d_m2lops
     size_t m2l_slots_at = 0;                        // the slot table in d_m2lops
-    size_t m2l_room = 0;         // bytes that C may take, where a buffer's reach is too little
-    bool m2l_short = false;      // the device had no room for more
+    size_t m2l_asked = 0, m2l_room = 0;  // bytes that the tree's C wants, and that the workspace may take (0: not asked yet)
+    size_t m2l_counted = 0;      // bytes of the workspace in the process's count
     int m2l_nrb = 0;             // row blocks of 16 (0: not prepared)
     std::vector<int> m2l_rboff;  // bytes of a target's C before each row block
     int m2l_variant = -1;    // M2L kernel variant; -1: pick by timing at the next M2L
@@ -295,6 +295,7 @@ int run_p2m(Context* c);
 int run_m2m(Context* c, int level);  // parents at `level`, children at level+1
 int prepare_m2l_f64(Context* c);  // tables and operator fragments of the uploaded operators (m2l_f64.hip)
 int run_m2l(Context* c);          // every level 2..h-1
+void count_m2l_workspace(Context* c);  // brings the process's count of workspaces up to date
 int run_l2l(Context* c, int level);  // parents at `level`
 int run_l2p(Context* c);
 int run_p2p(Context* c);

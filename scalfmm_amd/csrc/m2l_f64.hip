@@ -37,6 +37,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -529,7 +530,7 @@ __device__ __forceinline__ void down_body(const M2LArgs& a, const SmemLayout& sl
         rbd += 256 * n;
     }
     const double2* ops = reinterpret_cast<const double2*>(a.ops + static_cast<int64_t>(a.rb0) * rbd + wop) + lane;
-    d4* part = reinterpret_cast<d4*>(a.acc) + (static_cast<int64_t>(tile) * kMWaves + wave) * 4 * C * 64 + lane;
+    d4* part = reinterpret_cast<d4*>(a.acc) + (static_cast<int64_t>(tile) * kMWaves + wave) * K::nt(0) * C * 64 + lane;
     d4 acc[NT][C];
 #pragma unroll
     for (int t = 0; t < NT; ++t)
@@ -797,26 +798,34 @@ int pack_impl(Context* c, int nrb, const std::vector<char>& tables, size_t tau_a
     return check_launch(c, "m2l_pack");
 }
 
-// Device memory for C: all of it, or what kRoomMax and a quarter of the free
-// memory leave.  Beyond that the rows run in parts, each with the prologue of
-// every tile and with partial locals through memory (p^3 doubles per cell and
-// part).  Within a buffer's reach (4 GB) the upward kernel stores through a
-// buffer; beyond it with 64-bit addresses under a mask, which costs less than
-// the parts: 1M uniform h7, order 7 (12 GB) 17.2 ms in three parts, 16.4 in
-// one; 192 sets x 8 vectors, order 5, 51.0 / 48.5; 12M uniform h9, order 5, a
-// pass of 2,783 ms one step at a time, 730 with 32 GB, 530 with 64.
+// Device memory for C: all of it, or what kRoomMax and workspace_room leave.
+// Beyond that the rows run in parts, each with the prologue of every tile and
+// with partial locals through memory (p^3 doubles per cell and part).  Within a
+// buffer's reach (4 GB) the upward kernel stores through a buffer; beyond it
+// with 64-bit addresses under a mask, which costs less than the parts: 1M uniform
+// h7, order 7 (12 GB) 17.2 ms in three parts, 16.4 in one; 192 sets x 8 vectors,
+// order 5, 51.0 / 48.5; 12M uniform h9, order 5, a pass of 2,783 ms one step at a
+// time, 730 with 32 GB, 530 with 64.
 constexpr int kMaxPart = 116;  // row blocks of a launch: their table fits the LDS beside the tiles
 constexpr size_t kRoomMax = size_t(32) << 30;
 
-// Bytes that C may take of `want` (more than a buffer's reach).  The device is
-// asked only where a context wants more than before and got all of that, so that
-// a captured run decides as the run before it.
-size_t room_for_c(Context* c, size_t want) {
-    if (want > c->m2l_room && !c->m2l_short) {
-        size_t free_b = 0, total_b = 0;
-        if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) (void)hipGetLastError();
-        c->m2l_room = std::max(c->m2l_room, std::min(want, (free_b + c->d_m2lC.bytes) / 4));
-        c->m2l_short = c->m2l_room < want;
+// Bytes of the workspaces of the process on each device.
+std::atomic<size_t> g_held[64];
+
+// Bytes that the workspace may take of `want`.  The device is asked where a tree
+// wants more than before, and not again until the next build, so that a captured
+// run decides as the run before it and memory that was freed since then counts.
+size_t room_of(Context* c, size_t want) {
+    if (want > c->m2l_asked) {
+        c->m2l_asked = want;
+        const size_t own = c->d_m2lC.bytes + c->d_m2lacc.bytes;
+        if (c->d_m2lC.bytes >= want) {
+            c->m2l_room = want;
+        } else {
+            size_t free_b = 0, total_b = 0;
+            if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) (void)hipGetLastError();
+            c->m2l_room = workspace_room(want, own, std::max(own, g_held[c->device].load()), free_b);
+        }
     }
     return std::min(want, c->m2l_room);
 }
@@ -831,30 +840,28 @@ inline bool two_tiles(int64_t ncell) {
     return 17 * two < 10 * one;
 }
 
+// acc: bytes of the partial locals
 template <int P, int C, bool WIDE>
-int m2l_launch(Context* c, M2LArgs a, size_t room) {
+int m2l_launch(Context* c, M2LArgs a, size_t acc, size_t room) {
     using K = Cls<P>;
     constexpr int RB = Lds<C>::RB;
-    const int nrb = c->m2l_nrb;
     const int64_t tiles = (a.ncell + 16 * C - 1) / (16 * C);
     const int64_t grid = (tiles + 8 * kXcdChunk - 1) / (8 * kXcdChunk) * (8 * kXcdChunk);
-    // parts of the rows: whole steps, C within the workspace
-    std::vector<int> cut{0};
-    int64_t stride = 0;
-    while (cut.back() < nrb) {
-        int e = cut.back() + RB;
-        auto width = [&](int to) { return c->m2l_rboff[to] - c->m2l_rboff[cut.back()]; };
-        while (e < nrb && e + RB - cut.back() <= kMaxPart &&
-               static_cast<size_t>(width(std::min(e + RB, nrb))) * a.ncell <= room) e += RB;
-        e = std::min(e, nrb);
-        stride = std::max<int64_t>(stride, width(e));
-        cut.push_back(e);
+    std::vector<int> cut;
+    int parts = 0;
+    for (;;) {  // where the device refuses, smaller parts
+        const size_t bytes = cut_rows(c->m2l_rboff, RB, kMaxPart, a.ncell, acc, room, cut);
+        parts = static_cast<int>(cut.size()) - 1;
+        int st = parts > 1 ? ensure(c, c->d_m2lacc, acc) : HFMM_OK;
+        if (st == HFMM_OK) st = ensure(c, c->d_m2lC, bytes);
+        count_m2l_workspace(c);
+        if (st == HFMM_OK) break;
+        if (st != HFMM_ERR_NOMEM || parts * RB >= c->m2l_nrb) return st;
+        HFMM_HIP(c, hipStreamSynchronize(c->stream));
+        release(c->d_m2lC);
+        c->m2l_room = room = (bytes + (parts > 1 ? acc : 0)) / 2;
     }
-    HFMM_TRY(ensure(c, c->d_m2lC, static_cast<size_t>(stride) * a.ncell));
     a.C = c->d_m2lC.as<double>();
-    const int parts = static_cast<int>(cut.size()) - 1;
-    if (parts > 1)
-        HFMM_TRY(ensure(c, c->d_m2lacc, sizeof(double) * static_cast<size_t>(tiles) * kMWaves * 4 * C * 256));
     a.acc = c->d_m2lacc.as<double>();
     int maxrows = 0;
     for (int i = 0; i < parts; ++i) maxrows = std::max(maxrows, 16 * (cut[i + 1] - cut[i]));
@@ -903,11 +910,12 @@ int m2l_impl(Context* c) {
     a.slot_tau = reinterpret_cast<const uint16_t*>(c->d_m2lops.as<char>() + c->m2l_slots_at);
     int step = 0;
     for (int b = 0; b < c->m2l_nrb; ++b) step = std::max(step, c->m2l_rboff[b + 1] - c->m2l_rboff[b]);
-    const size_t all = std::min(static_cast<size_t>(c->m2l_rboff[c->m2l_nrb]) * a.ncell, kRoomMax);
-    const size_t room = all > kBufferMax ? room_for_c(c, all) : 0;
-    if (room > kBufferMax) return m2l_launch<P, 2, true>(c, a, room);
-    if (static_cast<size_t>(step) * a.ncell > kBufferMax) return m2l_launch<P, 2, true>(c, a, kBufferMax);
-    return two_tiles(a.ncell) ? m2l_launch<P, 2, false>(c, a, kBufferMax) : m2l_launch<P, 1, false>(c, a, kBufferMax);
+    const size_t all = static_cast<size_t>(c->m2l_rboff[c->m2l_nrb]) * a.ncell;
+    const size_t acc = sizeof(double) * 256 * Cls<P>::nt(0) * kMWaves * 2 * static_cast<size_t>((a.ncell + 31) / 32);
+    const bool parts = all > kRoomMax || c->m2l_nrb > kMaxPart;
+    const size_t room = room_of(c, std::min(all, kRoomMax) + (parts ? acc : 0));
+    if (room > kBufferMax || static_cast<size_t>(step) * a.ncell > kBufferMax) return m2l_launch<P, 2, true>(c, a, acc, room);
+    return two_tiles(a.ncell) ? m2l_launch<P, 2, false>(c, a, acc, room) : m2l_launch<P, 1, false>(c, a, acc, room);
 }
 
 #define HFMM_DISPATCH(P_, CALL)                                                   \
@@ -976,6 +984,13 @@ int prepare_m2l_f64(Context* c) {
     HFMM_TRY(pack());
     c->m2l_nrb = nrb;  // prepared: not before the memory is there and the kernel on its way
     return HFMM_OK;
+}
+
+void count_m2l_workspace(Context* c) {
+    const size_t now = c->d_m2lC.bytes + c->d_m2lacc.bytes;
+    if (now == c->m2l_counted) return;
+    g_held[c->device] += now - c->m2l_counted;  // modulo 2^64
+    c->m2l_counted = now;
 }
 
 int run_m2l(Context* c) {

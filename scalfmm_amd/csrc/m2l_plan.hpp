@@ -2,6 +2,7 @@
 // products and their places in a target's compressed expansions C.
 #pragma once
 
+#include <algorithm>
 #include <cstddef>
 #include <cstdint>
 #include <vector>
@@ -67,6 +68,42 @@ inline void row_layout(const TauInfo (&tau)[kTau], int nrb, std::vector<RowInfo>
     rboff[nrb] = off;
     for (RowInfo& ri : rows)
         if (ri.tau == kTauDummy) ri.off = static_cast<uint32_t>(off);
+}
+
+// Bytes that a context's workspace may take of `want`, with free_bytes left on the
+// device, `own` bytes in the context's workspace and `held` in all workspaces of the
+// process there: what it has, and its share of a quarter of the memory that is
+// free or in workspaces, so that several contexts together leave three
+// quarters to everything else.  Where that quarter is used up, a quarter of what
+// is free up to kRoomMin or a sixteenth of `want`: 16 parts at most.
+constexpr size_t kRoomMin = size_t(256) << 20;
+
+inline size_t workspace_room(size_t want, size_t own, size_t held, size_t free_bytes) {
+    const size_t quarter = (free_bytes + held) / 4, others = held - own;
+    size_t room = std::max(own, quarter > others ? quarter - others : 0);
+    room = std::max(room, std::min(std::max(want / 16, kRoomMin), (free_bytes + own) / 4));
+    return std::min(want, room);
+}
+
+// The rows in parts of whole steps (`step` row blocks): part i is row blocks cut[i] ..
+// cut[i + 1] - 1.  All in one part where their C fits `room` and a launch takes
+// max_part row blocks, else parts whose C fits beside acc_bytes of partial locals,
+// of one step at least.  Returns the bytes of C.
+inline size_t cut_rows(const std::vector<int>& rboff, int step, int max_part, int64_t ncell, size_t acc_bytes, size_t room,
+                       std::vector<int>& cut) {
+    const int nrb = static_cast<int>(rboff.size()) - 1;
+    const auto bytes = [&](int from, int to) { return static_cast<size_t>(rboff[to] - rboff[from]) * ncell; };
+    if (nrb > max_part || bytes(0, nrb) > room) room = room > acc_bytes ? room - acc_bytes : 0;
+    cut.assign(1, 0);
+    size_t most = 0;
+    while (cut.back() < nrb) {
+        const int b = cut.back();
+        int e = std::min(b + step, nrb);
+        while (e < nrb && e + step - b <= max_part && bytes(b, std::min(e + step, nrb)) <= room) e = std::min(e + step, nrb);
+        most = std::max(most, bytes(b, e));
+        cut.push_back(e);
+    }
+    return most;
 }
 
 }  // namespace hfmm

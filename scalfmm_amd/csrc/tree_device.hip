@@ -1024,6 +1024,7 @@ int build_tree_device(Context* c) {
     c->evaluated = false;
     c->p2p_mutual = false;
     c->order_built = false;
+    c->m2l_asked = 0;
     if (c->p2p_items_cap > 0) HFMM_TRY(build_p2p_mutual_tables(c, nbig));
     return HFMM_OK;
 }

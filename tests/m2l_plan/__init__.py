@@ -19,6 +19,11 @@ def lib():
     L = ctypes.CDLL(out)
     tmp.cleanup()  # the loaded library stays
     L.plan_nowhere.restype = ctypes.c_uint32
+    L.plan_room.restype = ctypes.c_uint64
+    L.plan_room.argtypes = [ctypes.c_uint64] * 4
+    L.plan_cut.restype = ctypes.c_uint64
+    L.plan_cut.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int64, ctypes.c_uint64,
+                           ctypes.c_uint64, ctypes.c_void_p, ctypes.c_void_p]
     return L
 
 
@@ -30,3 +35,13 @@ def rows(rank):
     nrb = lib().plan_rows(*(a.ctypes.data_as(ctypes.c_void_p) for a in (rank, tau, off, last, rboff)))
     n = 16 * nrb
     return tau[:n], off[:n], last[:n], rboff[: nrb + 1]
+
+
+def cut(rboff, step, max_part, ncell, acc, room):
+    """(first row blocks of the parts and the end, bytes of C)"""
+    rboff = np.ascontiguousarray(rboff, np.int32)
+    out = np.zeros(len(rboff) + 1, np.int32)
+    parts = ctypes.c_int()
+    size = lib().plan_cut(rboff.ctypes.data, len(rboff) - 1, step, max_part, ncell, acc, room, out.ctypes.data,
+                          ctypes.addressof(parts))
+    return out[: parts.value + 1], size

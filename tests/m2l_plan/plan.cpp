@@ -34,4 +34,18 @@ int plan_rows(const int32_t* rank, uint32_t* tau_of, uint32_t* off, uint32_t* la
     return nrb;
 }
 
+uint64_t plan_room(uint64_t want, uint64_t own, uint64_t held, uint64_t free_bytes) {
+    return workspace_room(want, own, held, free_bytes);
+}
+
+// Parts of the rows: their first row blocks into cut, and the end; the bytes of C.
+uint64_t plan_cut(const int32_t* rboff, int nrb, int step, int max_part, int64_t ncell, uint64_t acc, uint64_t room,
+                  int32_t* cut, int* parts) {
+    std::vector<int> c;
+    const uint64_t bytes = cut_rows(std::vector<int>(rboff, rboff + nrb + 1), step, max_part, ncell, acc, room, c);
+    for (size_t i = 0; i < c.size(); ++i) cut[i] = c[i];
+    *parts = static_cast<int>(c.size()) - 1;
+    return bytes;
+}
+
 }  // extern "C"

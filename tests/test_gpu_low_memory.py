@@ -39,3 +39,41 @@ def test_products_prepared_again_after_a_failure():
         assert np.array_equal(a, b)
     e.close()
     ref.close()
+
+
+@pytest.mark.parametrize("n,h,order,cells,left", [(60000, 6, 7, (28000, 37449), 900 << 20), (9000, 6, 8, (8193, 12288), 300 << 20),
+                                                  (60000, 6, 5, (28000, 37449), 400 << 20)])
+def test_fp64_m2l_with_little_memory(n, h, order, cells, left):
+    """The compressed expansions (0.6 to 1.3 GB here) find less memory than
+    they would take: the rows run in parts, with the same bits, and all at once
+    again when the memory is back."""
+    from device_memory import all_but
+    from scalfmm_amd import Engine, FFmmM2L, FFmmNearAndFarFields
+    from scalfmm_amd.distributions import uniform_cube
+    x, y, z, q = uniform_cube(n, 7)
+
+    def engine():
+        e = Engine(h, 1.0, CENTER, order)
+        e.set_particles(x, y, z, q)
+        e.build_tree()
+        assert cells[0] <= sum(e.tree_info().n_cells) <= cells[1]  # the tile shape
+        return e
+
+    e = engine()
+    e.evaluate()
+    ref = e.results()
+    e.close()
+    e = engine()
+    e.evaluate(FFmmNearAndFarFields & ~FFmmM2L)  # every other buffer
+    e.synchronize()
+    with all_but(left) as free:
+        print("left", free, flush=True)
+        for _ in range(2):
+            e.evaluate()
+            for a, b in zip(e.results(), ref):
+                assert np.array_equal(a, b)
+    e.build_tree()
+    e.evaluate()
+    for a, b in zip(e.results(), ref):
+        assert np.array_equal(a, b)
+    e.close()
