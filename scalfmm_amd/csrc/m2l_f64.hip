@@ -830,16 +830,6 @@ size_t room_of(Context* c, size_t want) {
     return std::min(want, c->m2l_room);
 }
 
-// Two column tiles per workgroup (32 cells) reuse the operators but take 1.7
-// times as long as one (1,000 uniform particles, order 7: 354 against 205 us), so
-// they pay where they need fewer rounds of the 256 CUs: 585 cells, order 8, 575
-// against 338 us; 4,681 cells, order 5 139 / 154, order 8 595 / 711; 37,449 cells,
-// order 6 1,239 / 1,400.
-inline bool two_tiles(int64_t ncell) {
-    const int64_t one = (ncell + 16 * 256 - 1) / (16 * 256), two = (ncell + 32 * 256 - 1) / (32 * 256);
-    return 17 * two < 10 * one;
-}
-
 // acc: bytes of the partial locals
 template <int P, int C, bool WIDE>
 int m2l_launch(Context* c, M2LArgs a, size_t acc, size_t room) {

@@ -70,6 +70,16 @@ inline void row_layout(const TauInfo (&tau)[kTau], int nrb, std::vector<RowInfo>
         if (ri.tau == kTauDummy) ri.off = static_cast<uint32_t>(off);
 }
 
+// Two column tiles per workgroup (32 cells) reuse the operators but take 1.7
+// times as long as one (1,000 uniform particles, order 7: 354 against 205 us), so
+// they pay where they need fewer rounds of the 256 CUs: 585 cells, order 8, 575
+// against 338 us; 4,681 cells, order 5 139 / 154, order 8 595 / 711; 37,449 cells,
+// order 6 1,239 / 1,400.
+inline bool two_tiles(int64_t ncell) {
+    const int64_t one = (ncell + 16 * 256 - 1) / (16 * 256), two = (ncell + 32 * 256 - 1) / (32 * 256);
+    return 17 * two < 10 * one;
+}
+
 // Bytes that a context's workspace may take of `want`, with free_bytes left on the
 // device, `own` bytes in the context's workspace and `held` in all workspaces of the
 // process there: what it has, and its share of a quarter of the memory that is

@@ -19,12 +19,18 @@ def lib():
     L = ctypes.CDLL(out)
     tmp.cleanup()  # the loaded library stays
     L.plan_nowhere.restype = ctypes.c_uint32
+    L.plan_two_tiles.argtypes = [ctypes.c_int64]
     L.plan_room.restype = ctypes.c_uint64
     L.plan_room.argtypes = [ctypes.c_uint64] * 4
     L.plan_cut.restype = ctypes.c_uint64
     L.plan_cut.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int64, ctypes.c_uint64,
                            ctypes.c_uint64, ctypes.c_void_p, ctypes.c_void_p]
     return L
+
+
+def two_tiles(ncell):
+    """Whether a workgroup takes two column tiles (32 cells)."""
+    return bool(lib().plan_two_tiles(int(ncell)))
 
 
 def rows(rank):

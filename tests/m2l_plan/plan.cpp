@@ -34,6 +34,8 @@ int plan_rows(const int32_t* rank, uint32_t* tau_of, uint32_t* off, uint32_t* la
     return nrb;
 }
 
+int plan_two_tiles(int64_t ncell) { return two_tiles(ncell); }
+
 uint64_t plan_room(uint64_t want, uint64_t own, uint64_t held, uint64_t free_bytes) {
     return workspace_room(want, own, held, free_bytes);
 }
