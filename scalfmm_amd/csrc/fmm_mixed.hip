@@ -997,6 +997,11 @@ int m2l_mixed_impl(Context* c) {
 
 }  // namespace
 
+bool variant_takes_tiles(const Context* c, int v) {
+    return is_mixed(c) && (v < 0 ? c->order() < kF64ProductsOrder : v < kMixedVariants);
+}
+bool tiles_by_default(const Context* c) { return variant_takes_tiles(c, -1); }
+
 int prepare_mixed_operators(Context* c) {
     const ChebOperators& op = c->ops;
     const int LD = c->LD;
@@ -1045,6 +1050,7 @@ int prepare_mixed_operators(Context* c) {
             HFMM_TRY(check_launch(c, "pack_positions"));
         }
         HFMM_HIP(c, hipStreamSynchronize(c->stream));
+        c->mixed_ready = true;
         return HFMM_OK;
     };
     const int st = run();
@@ -1065,6 +1071,7 @@ int run_split_multipoles(Context* c) {
 
 int run_m2l_mixed(Context* c) {
     if (c->kpad_max > 64) return fail(c, HFMM_ERR_ARG, "operator rank above 64 is not supported");
+    if (!c->mixed_ready) HFMM_TRY(prepare_mixed_operators(c));
     HFMM_TRY(ensure_parity_order(c));
     // three-part splits (six products) or, in HFMM_PRECISION_MIXED_HILO, two-part
     // hi/lo splits (three products)

@@ -197,6 +197,7 @@ static int upload_operators(Context* c) {
     HFMM_TRY(ensure(c, c->d_slotseg, sizeof(int32_t) * seg.size()));
     HFMM_HIP(c, hipMemcpy(c->d_slotseg.ptr, seg.data(), sizeof(int32_t) * seg.size(), hipMemcpyHostToDevice));
     c->m2l_nrb = 0;
+    c->mixed_ready = false;
     return is_mixed(c) ? HFMM_OK : prepare_m2l_f64(c);
 }
 
@@ -310,7 +311,7 @@ int create_context(const hfmm_params* params, hipStream_t shared_stream, hfmm_ct
     if (st == HFMM_OK && scheme == HFMM_M2L_SYMMETRIC) st = hfmm::compress_operators_device(c);
     c->sym_compressed = c->sym_uploaded = scheme == HFMM_M2L_SYMMETRIC;
     if (st == HFMM_OK) st = hfmm::upload_operators(c);  // rank-0 operators until compressed
-    if (st == HFMM_OK && hfmm::is_mixed(c)) st = hfmm::prepare_mixed_operators(c);
+    if (st == HFMM_OK && hfmm::tiles_by_default(c)) st = hfmm::prepare_mixed_operators(c);
     if (st == HFMM_OK && scheme != HFMM_M2L_SYMMETRIC) st = hfmm_set_m2l_scheme(h, scheme);
     if (st != HFMM_OK) {
         hfmm::free_all(c);
@@ -862,7 +863,7 @@ int hfmm_load_operators(hfmm_ctx* h, const char* path) {
         HFMM_TRY(hfmm::upload_operators(c));
         c->sym_uploaded = true;
     }
-    if (hfmm::is_mixed(c)) HFMM_TRY(hfmm::prepare_mixed_operators(c));
+    if (hfmm::tiles_by_default(c)) HFMM_TRY(hfmm::prepare_mixed_operators(c));
     c->m2l_variant = -1;  // other operators: tune again
     c->evaluated = false;
     return HFMM_OK;
@@ -1027,6 +1028,10 @@ int hfmm_set_m2l_variant(hfmm_ctx* h, int32_t variant) {
     Context* c = &h->c;
     if (variant != -1 && !hfmm::m2l_variant_available(c, variant))
         return hfmm::fail(c, HFMM_ERR_ARG, "M2L variant not available for this order and precision");
+    if (hfmm::variant_takes_tiles(c, variant) && !c->mixed_ready) {
+        HFMM_HIP(c, hipSetDevice(c->device));
+        HFMM_TRY(hfmm::prepare_mixed_operators(c));
+    }
     c->m2l_variant = variant;
     return HFMM_OK;
 }

@@ -101,6 +101,7 @@ struct Context {
     size_t m2l_counted = 0;      // bytes of the workspace in the process's count
     int m2l_nrb = 0;             // row blocks of 16 (0: not prepared)
     std::vector<int> m2l_rboff;  // bytes of a target's C before each row block
+    bool mixed_ready = false;  // d_opm and d_opm2 hold the uploaded operators
     int m2l_variant = -1;    // M2L kernel variant; -1: pick by timing at the next M2L
     float m2l_tune_ms[4] = {0.f, 0.f, 0.f, 0.f};  // times measured by the last autotune
 
@@ -343,6 +344,10 @@ int selftest_mfma_f64(Context* c, double* out);
 
 // Mixed-precision passes (fmm_mixed.hip)
 int prepare_mixed_operators(Context* c);  // position-specific bf16 operators
+// Whether a context of variant v runs the bfloat16 tiles, and so needs their
+// operators (108 MB and 10 ms at order 8); whether one does whose variant is not set.
+bool variant_takes_tiles(const Context* c, int v);
+bool tiles_by_default(const Context* c);
 int run_split_multipoles(Context* c);     // d_M -> d_Mb
 int run_m2l_mixed(Context* c);
 int run_p2p_mixed(Context* c);
