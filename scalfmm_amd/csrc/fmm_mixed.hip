@@ -166,7 +166,7 @@ __global__ __launch_bounds__(256) void k_modal_to_nodal(int64_t ncells, const do
     __shared__ double buf[4][2][NN];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     for (int i = threadIdx.x; i < P * P; i += 256) sT[i] = Troots[i];
-    const int64_t cell = static_cast<int64_t>(blockIdx.x) * 4 + wave;
+    const int64_t cell = thread_of_grid256() >> 6;
     const bool live = cell < ncells;
     double* Lc = L + (live ? cell : 0) * LD;
     double* a = buf[wave][0];
@@ -198,7 +198,7 @@ __global__ __launch_bounds__(256) void k_modal_to_nodal(int64_t ncells, const do
 // each value into three bfloat16 parts in registers as it loads it.
 __global__ __launch_bounds__(256) void k_split_multipoles(int64_t nvals, const double* __restrict__ M,
                                                          float* __restrict__ Mf) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    const int64_t i = thread_of_grid256();
     if (i >= nvals) return;
     Mf[i] = static_cast<float>(M[i]);
 }
@@ -879,6 +879,7 @@ int m2l_mixed_launch(Context* c) {
     int tiles = 0;
     const M2LLevels lv = make_levels(c, 16 * COLS, tiles);
     if (tiles == 0) return HFMM_OK;  // no M2L level in the working range
+    if (tiles >= 1 << 24) return fail(c, HFMM_ERR_ARG, "mixed M2L: more cells than one launch of this shape holds");
     const int CR = ((c->kpad_max + 31) & ~31) + 4;
     const size_t shmem = sizeof(float) * kM2LWaves * static_cast<size_t>(CR) * 16 * COLS + 16 * COLS * 2 * 3 * 64;
     static int lds_limit[64] = {0};
@@ -989,7 +990,7 @@ int m2l_mixed_impl(Context* c) {
     // the M2L targets: every cell of levels top..h-1, contiguous in the cell arrays
     const int64_t first = c->lvl_off[c->top()], ncells = c->lvl_off[c->height()] - first;
     prof_begin(c, "modal_to_nodal");
-    hipLaunchKernelGGL(k_modal_to_nodal<P>, dim3(static_cast<unsigned>((ncells + 3) / 4)), dim3(256), 0, c->stream,
+    hipLaunchKernelGGL(k_modal_to_nodal<P>, grid256(64 * ncells), dim3(256), 0, c->stream,
                        ncells, c->d_Troots.as<double>(), c->d_L.as<double>() + first * c->LD, c->LD);
     prof_end(c);
     return check_launch(c, "modal_to_nodal");
@@ -1063,7 +1064,7 @@ int run_split_multipoles(Context* c) {
     const int64_t nvals = (c->total_cells + 1) * static_cast<int64_t>(c->LD);
     HFMM_TRY(ensure(c, c->d_Mb, sizeof(float) * static_cast<size_t>(nvals)));
     prof_begin(c, "split_multipoles");
-    hipLaunchKernelGGL(k_split_multipoles, dim3(blocks_of(nvals)), dim3(256), 0, c->stream, nvals,
+    hipLaunchKernelGGL(k_split_multipoles, grid256(nvals), dim3(256), 0, c->stream, nvals,
                        c->d_M.as<double>(), c->d_Mb.as<float>());
     prof_end(c);
     return check_launch(c, "split_multipoles");

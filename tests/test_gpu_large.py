@@ -1,6 +1,5 @@
-"""More than 2^29 particles: eight lanes each are more threads than one dimension
-of a launch holds.  The near field of a few targets, the last of the sorted order
-among them, against sums over their 27 leaves (1e-12, the FP64 path's bound)."""
+"""Sizes at which a kernel needs more threads than one dimension of a launch
+holds (2^32)."""
 import ctypes
 
 import pytest
@@ -11,6 +10,9 @@ N, H = (1 << 29) + 4099, 9
 
 
 def test_near_field_beyond_2_29_particles():
+    """Eight lanes per particle.  The near field of a few targets, the last of the
+    Morton order among them, against sums over their 27 leaves (1e-12, the FP64
+    path's bound)."""
     import torch
     from scalfmm_amd import Engine, FFmmNearField
     if torch.cuda.mem_get_info()[0] < 220 << 30:
@@ -47,4 +49,49 @@ def test_near_field_beyond_2_29_particles():
         assert abs(float(got[i] - want)) <= 1e-12 * float(want), i
     e.close()
     del got, pos, q, near, at
+    torch.cuda.empty_cache()
+
+
+def test_mixed_multipoles_beyond_2_32():
+    """52 million cells of 128 multipoles at order 5 in the hi/lo form: potentials
+    of targets at both ends of the Morton order against direct sums, within the
+    order's interpolation error (1e-3, as on the smaller sets, and a factor of ten)."""
+    import torch
+    from scalfmm_amd import PRECISION_MIXED_HILO, Engine
+    if torch.cuda.mem_get_info()[0] < 240 << 30:
+        pytest.skip("needs 240 GiB of device memory")
+    n, h = 40_000_003, 10
+    g = torch.Generator(device="cuda")
+    g.manual_seed(12)
+    pos = [torch.rand(n, generator=g, device="cuda", dtype=torch.float64) for _ in range(3)]
+    q = 2 * torch.rand(n, generator=g, device="cuda", dtype=torch.float64) - 1
+    for d in range(3):
+        pos[d][:32] *= 0.01
+        pos[d][32:64] = 1 - 0.01 * pos[d][32:64]
+    torch.cuda.synchronize()
+    e = Engine(h, 1.0, (0.5, 0.5, 0.5), 5, precision=PRECISION_MIXED_HILO)
+    e.set_m2l_variant(2)
+    e.set_particles_device(n, *(a.data_ptr() for a in (*pos, q)))
+    e.build_tree()
+    e.evaluate()
+    e.synchronize()
+    p = ctypes.c_void_p()
+    assert e._L.hfmm_get_results_device(e.h, ctypes.byref(p), None, None, None) == 0
+
+    class Block:
+        __cuda_array_interface__ = {"data": (p.value, False), "shape": (n,), "typestr": "<f8", "version": 3}
+
+    got = torch.as_tensor(Block(), device="cuda")
+    for t in (range(32), range(32, 64)):
+        want = []
+        for i in t:
+            r2 = sum((a - a[i]) ** 2 for a in pos)
+            r2[i] = float("inf")
+            want.append((q * r2.rsqrt()).sum())
+        want = torch.stack(want)
+        err = float((got[t.start:t.stop] - want).norm() / want.norm())
+        print(f"targets {t}: {err:.2e}", flush=True)
+        assert err <= 1e-2
+    e.close()
+    del got, pos, q, r2
     torch.cuda.empty_cache()
