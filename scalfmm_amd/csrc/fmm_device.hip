@@ -783,8 +783,8 @@ __device__ __forceinline__ void p2p_f64_mutual_item(const int32_t* __restrict__ 
     }
 }
 
-__global__ __launch_bounds__(256) void k_p2p_f64_mutual(const int2* __restrict__ items, const int32_t* __restrict__ nitems,
-                                                       const int32_t* __restrict__ lstart,
+__global__ __launch_bounds__(256) void k_p2p_f64_mutual(const int2* __restrict__ items, const int32_t* __restrict__ claims,
+                                                       int total, const int32_t* __restrict__ lstart,
                                                        const int32_t* __restrict__ slots, const double* __restrict__ sp,
                                                        int64_t n, const int32_t* __restrict__ csoff,
                                                        const int64_t* __restrict__ csbase,
@@ -794,21 +794,19 @@ __global__ __launch_bounds__(256) void k_p2p_f64_mutual(const int2* __restrict__
     __shared__ double2 s_xy[4][128], s_zq[4][128];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int total = *nitems;
-    // parts of work items claimed one at a time, costliest items first (kP2PMaxParts
-    // claims each, most items have one part); every wave leaves once the counter
-    // passes the last
+    // parts of work items claimed one at a time, costliest items first; every wave
+    // leaves once the counter passes the last
     for (;;) {
-        int claim = 0;
-        if (lane == 0) claim = atomicAdd(next, 1);
-        const int at = __builtin_amdgcn_readfirstlane(__shfl(claim, 0));
-        const int it = at / kP2PMaxParts, part = at % kP2PMaxParts;
-        if (it >= total) break;
-        const int2 item = items[it];
+        int at = 0;
+        if (lane == 0) at = atomicAdd(next, 1);
+        at = __builtin_amdgcn_readfirstlane(at);
+        if (at >= total) break;
+        const int claim = __builtin_amdgcn_readfirstlane(claims[at]);
+        const int part = claim % kP2PMaxParts;
+        const int2 item = items[claim / kP2PMaxParts];
         const int leaf = __builtin_amdgcn_readfirstlane(item.x);
         const int first = __builtin_amdgcn_readfirstlane(item.y);
         const int parts = __builtin_amdgcn_readfirstlane(csparts[leaf]);
-        if (part >= parts) continue;
         const int l0 = __builtin_amdgcn_readfirstlane(lstart[leaf]);
         const int tend = min(__builtin_amdgcn_readfirstlane(lstart[leaf + 1]), first + kP2PMutualItem);
         const int tile = (first - l0) / kP2PMutualItem;
@@ -1053,12 +1051,12 @@ int run_p2p(Context* c) {
             HFMM_HIP(c, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device));
             resident[c->device] = std::max(1, per_cu) * std::max(1, cus);
         }
-        const int64_t want = (c->p2p_items_m_cap * kP2PMaxParts + 3) / 4;
+        const int64_t want = (c->p2p_claims + 3) / 4;
         const unsigned grid = static_cast<unsigned>(std::max<int64_t>(1, std::min<int64_t>(want, resident[c->device])));
         HFMM_TRY(zero_device(c, p2p_mutual_next(c), sizeof(int32_t)));  // a fill kernel: capturable
         prof_begin(c, "p2p_big");
         hipLaunchKernelGGL(k_p2p_f64_mutual, dim3(grid), dim3(256), 0, c->stream, c->d_p2pitems_m.as<int2>(),
-                           p2p_mutual_item_count(c), c->d_leafstart.as<int32_t>(), c->d_p2p.as<int32_t>(),
+                           c->d_claims.as<int32_t>(), c->p2p_claims, c->d_leafstart.as<int32_t>(), c->d_p2p.as<int32_t>(),
                            c->d_sorted.as<double>(), c->n, c->d_csoff.as<int32_t>(), c->d_csbase.as<int64_t>(),
                            c->d_csparts.as<int32_t>(), c->d_cpart.as<d4>(), p2p_mutual_next(c), sorted_results(c));
         prof_end(c);

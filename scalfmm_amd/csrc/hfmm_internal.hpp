@@ -161,6 +161,8 @@ struct Context {
     int64_t p2p_items_m_cap = 0;
     DevBuf d_csoff;                           // int32 [nleaf][13]
     DevBuf d_csparts;                         // int32 [nleaf] parts of an item (FP64)
+    DevBuf d_claims;                          // int32 [p2p_claims] item kP2PMaxParts + part (FP64)
+    int32_t p2p_claims = 0;
     DevBuf d_csbase;                          // int64 [nleaf + 1]
     DevBuf d_direct;                          // staging of hfmm_direct
     DevBuf d_cpart;                           // source-side partial sums
@@ -281,9 +283,11 @@ inline int32_t* p2p_item_count(Context* c) { return reinterpret_cast<int32_t*>(c
 // its source-side partial sums (float4 entries).
 inline int32_t* p2p_mutual_item_count(Context* c) { return reinterpret_cast<int32_t*>(c->d_count.as<int64_t>() + 16); }
 inline int64_t* p2p_mutual_units(Context* c) { return c->d_count.as<int64_t>() + 17; }
-// The next work item of the mutual mixed P2P (claimed by the waves one at a
+// The number of claims of the mutual FP64 P2P, behind the units (both are read at once).
+inline int32_t* p2p_claim_count(Context* c) { return reinterpret_cast<int32_t*>(c->d_count.as<int64_t>() + 18); }
+// The next work item (claim) of the mutual P2P (taken by the waves one at a
 // time; cleared before each launch).
-inline int32_t* p2p_mutual_next(Context* c) { return reinterpret_cast<int32_t*>(c->d_count.as<int64_t>() + 18); }
+inline int32_t* p2p_mutual_next(Context* c) { return reinterpret_cast<int32_t*>(c->d_count.as<int64_t>() + 19); }
 // Builds the mutual P2P's work items and slot tables on a built tree and sizes
 // the partial buffer; leaves c->p2p_mutual false when the
 // partial sums would exceed a quarter of the free device memory.

@@ -819,6 +819,27 @@ __global__ __launch_bounds__(kBlock) void k_colslot_counts(int nleaf, const int3
     units[i] = static_cast<int64_t>(run + k - 1) * m;
 }
 
+// The claims of the FP64 kernel, item kP2PMaxParts + part, in the items' order
+// (costliest first): parts per item, then their places after a scan.  Claims of
+// kP2PMaxParts parts for every item, most of them empty, came to 3.3 ns per item
+// and part on the one counter: 4.1 of the 8.2 ms of 2M uniform particles at height
+// 6 (10,562 items).
+__global__ __launch_bounds__(kBlock) void k_item_parts(int64_t cap, const int32_t* __restrict__ nitems,
+                                                      const int2* __restrict__ items, const int32_t* __restrict__ parts,
+                                                      int32_t* __restrict__ cnt) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i < cap) cnt[i] = i < *nitems ? parts[items[i].x] : 0;
+}
+
+__global__ __launch_bounds__(kBlock) void k_item_claims(int64_t cap, const int32_t* __restrict__ nitems,
+                                                       const int2* __restrict__ items, const int32_t* __restrict__ parts,
+                                                       const int32_t* __restrict__ off, int32_t* __restrict__ claims) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i >= cap || i >= *nitems) return;
+    const int k = parts[items[i].x];
+    for (int p = 0; p < k; ++p) claims[off[i] + p] = static_cast<int32_t>(i) * kP2PMaxParts + p;
+}
+
 }  // namespace
 
 int m2l_slot_counts(Context* c, int level, unsigned long long* counts) {
@@ -1089,9 +1110,20 @@ int build_p2p_mutual_tables(Context* c, int64_t nbig) {
     prof_end(c);
     HFMM_TRY(check_launch(c, "p2p_items"));
     HFMM_TRY(exclusive_scan<int64_t>(c, base, base, nl, p2p_mutual_units(c), "p2p_items"));
-    int64_t units = 0;
-    HFMM_HIP(c, hipMemcpyAsync(&units, p2p_mutual_units(c), sizeof(int64_t), hipMemcpyDeviceToHost, c->stream));
+    const int64_t cap = c->p2p_items_m_cap;
+    if (!is_mixed(c)) {
+        HFMM_TRY(ensure(c, c->d_scan, sizeof(int32_t) * static_cast<size_t>(cap)));
+        prof_begin(c, "p2p_items");
+        hipLaunchKernelGGL(k_item_parts, dim3(blocks_for(cap)), dim3(kBlock), 0, c->stream, cap, p2p_mutual_item_count(c),
+                           c->d_p2pitems_m.as<int2>(), c->d_csparts.as<int32_t>(), c->d_scan.as<int32_t>());
+        prof_end(c);
+        HFMM_TRY(check_launch(c, "p2p_items"));
+        HFMM_TRY(exclusive_scan<int32_t>(c, c->d_scan.as<int32_t>(), c->d_scan.as<int32_t>(), cap, p2p_claim_count(c), "p2p_items"));
+    }
+    int64_t counts[2] = {0, 0};  // units, claims
+    HFMM_HIP(c, hipMemcpyAsync(counts, p2p_mutual_units(c), sizeof(counts), hipMemcpyDeviceToHost, c->stream));
     HFMM_HIP(c, hipStreamSynchronize(c->stream));
+    const int64_t units = counts[0];
     // base[nl] = the total, so a leaf's slot count is (base[i+1] - base[i]) / n_i
     HFMM_HIP(c, hipMemcpyAsync(base + nl, p2p_mutual_units(c), sizeof(int64_t), hipMemcpyDeviceToDevice, c->stream));
     const size_t bytes = (is_mixed(c) ? sizeof(float) : sizeof(double)) * 4 * static_cast<size_t>(units > 0 ? units : 1);
@@ -1101,6 +1133,16 @@ int build_p2p_mutual_tables(Context* c, int64_t nbig) {
         if (bytes > (free_b + c->d_cpart.bytes) / 4) return HFMM_OK;  // ordered-pair kernel instead
     }
     HFMM_TRY(ensure(c, c->d_cpart, bytes));
+    if (!is_mixed(c)) {
+        c->p2p_claims = static_cast<int32_t>(counts[1]);
+        HFMM_TRY(ensure(c, c->d_claims, sizeof(int32_t) * static_cast<size_t>(c->p2p_claims)));
+        prof_begin(c, "p2p_items");
+        hipLaunchKernelGGL(k_item_claims, dim3(blocks_for(cap)), dim3(kBlock), 0, c->stream, cap, p2p_mutual_item_count(c),
+                           c->d_p2pitems_m.as<int2>(), c->d_csparts.as<int32_t>(), c->d_scan.as<int32_t>(),
+                           c->d_claims.as<int32_t>());
+        prof_end(c);
+        HFMM_TRY(check_launch(c, "p2p_items"));
+    }
     c->cpart_units = units;
     c->p2p_mutual = true;
     return HFMM_OK;
