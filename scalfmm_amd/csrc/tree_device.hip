@@ -777,16 +777,21 @@ int sort_p2p_items(Context* c, int2* items, const int32_t* nitems, int64_t cap) 
 // neighbour in slot 25 - s.  Per big leaf B: the 13 offsets (one per backward
 // slot 13..25, -1 when that neighbour is absent or small) and units[B] =
 // (number of slots) x (particles of B) entries.
-// An item of the FP64 kernel is taken in parts[A] parts of about kP2PPartPairs
+// An item of the FP64 kernel is taken in parts[A] parts of about part_pairs
 // pairs, each a range of the sources of A itself and of its big forward
 // neighbours: one wave would need 14 ms for a central item of a Plummer set of
 // 120,000 particles at height 6 (256 targets, 70,000 sources).  Part 0 writes
 // the targets' results, each further part a slot of A's own, after those of the
-// backward neighbours.
-constexpr int64_t kP2PPartPairs = int64_t(1) << 18;
+// backward neighbours.  Few items leave most of the 4,096 waves idle behind the
+// longest ones, so that they go in parts of 2^14 pairs, a chunk or two of 64
+// sources: near field with its combination in us, 2^14 / 2^18 / ordered pairs: 8
+// items (3,000 Plummer, h6) 101 / 220 / 133; 256 (30,000 on a line, h9) 51 / 78 / 50;
+// about 700 (120k Plummer, h6) 1,450 / 1,652 / 4,914; 2,500 (400k Plummer, h7)
+// 2,842 / 3,066 / 8,739; 8,000 (1M uniform, h5) 3,781 / 3,470 / 5,428.
+inline int64_t part_pairs(int64_t items) { return int64_t(1) << (items <= 4096 ? 14 : 18); }
 
 __global__ __launch_bounds__(kBlock) void k_colslot_counts(int nleaf, const int32_t* __restrict__ lstart,
-                                                           const int32_t* __restrict__ slots, int split,
+                                                           const int32_t* __restrict__ slots, int64_t part_pairs,
                                                            int32_t* __restrict__ csoff, int64_t* __restrict__ units,
                                                            int32_t* __restrict__ parts) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -806,14 +811,14 @@ __global__ __launch_bounds__(kBlock) void k_colslot_counts(int nleaf, const int3
         csoff[static_cast<int64_t>(i) * kNbrForward + b] = o;
     }
     int k = 1;
-    if (split && m > kP2PBig) {
+    if (part_pairs && m > kP2PBig) {
         int64_t src = m;
         for (int b = 0; b < kNbrForward; ++b) {
             const int a = slots[static_cast<int64_t>(i) * kNbrSlots + b];
             const int na = a < 0 ? 0 : lstart[a + 1] - lstart[a];
             if (na > kP2PBig) src += na;
         }
-        k = static_cast<int>(min(static_cast<int64_t>(kP2PMaxParts), 1 + src * min(m, kP2PMutualItem) / kP2PPartPairs));
+        k = static_cast<int>(min(static_cast<int64_t>(kP2PMaxParts), 1 + src * min(m, kP2PMutualItem) / part_pairs));
     }
     parts[i] = k;
     units[i] = static_cast<int64_t>(run + k - 1) * m;
@@ -1106,7 +1111,7 @@ int build_p2p_mutual_tables(Context* c, int64_t nbig) {
     int64_t* base = c->d_csbase.as<int64_t>();
     prof_begin(c, "p2p_items");
     hipLaunchKernelGGL(k_colslot_counts, dim3(blocks_for(nl)), dim3(kBlock), 0, c->stream, static_cast<int>(nl), lstart,
-                       c->d_p2p.as<int32_t>(), is_mixed(c) ? 0 : 1, c->d_csoff.as<int32_t>(), base, c->d_csparts.as<int32_t>());
+                       c->d_p2p.as<int32_t>(), is_mixed(c) ? 0 : part_pairs(c->p2p_items_m_cap), c->d_csoff.as<int32_t>(), base, c->d_csparts.as<int32_t>());
     prof_end(c);
     HFMM_TRY(check_launch(c, "p2p_items"));
     HFMM_TRY(exclusive_scan<int64_t>(c, base, base, nl, p2p_mutual_units(c), "p2p_items"));
