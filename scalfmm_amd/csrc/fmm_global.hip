@@ -339,18 +339,27 @@ struct UnifLevels {
 };
 constexpr int kUnifCells = 32;
 
-// L^ += scale K^_pos . M^[src] entrywise (FUnifM2LHandler::applyFC), every M2L
-// level in one launch.  A wave takes the siblings of one parent (up to 8
-// targets) and 64 spectrum entries: for each of the 26 neighbour parents it
-// reads the 8 source spectra once for all targets, and each of the 27 kernel
-// spectra of that direction (offset 2 d + b - a of source child b from target
-// child a, at most 3 values per axis) once for the 1 to 8 pairs that have it.
-// One target at a time, every pair reads both: 3,024 spectra for the 8 targets
+// L^ += scale K^_pos . M^[src] entrywise (FUnifM2LHandler::applyFC), the levels of
+// many children per parent in one launch (FULL), those of few in another.  A wave takes
+// the siblings of one parent (up to 8 targets) and 64 spectrum entries: for each
+// of the 26 neighbour parents FULL reads the 8 source spectra once for all
+// targets, and each of the 27 kernel spectra of that direction (offset 2 d + b - a
+// of source child b from target child a, at most 3 values per axis) once for the 1
+// to 8 pairs that have it.  One target at a time, every pair reads both: 3,024 spectra for the 8 targets
 // of a full parent against 910 here, and the caches were the bound (15.7 TB/s,
-// 2.13 ms at 20,000 particles, height 5, order 7).
+// 2.13 ms at 20,000 particles, height 5, order 7; 0.56 ms now).
 // A workgroup's four waves take the parents that begin in its kUnifCells cells,
 // so they read the same kernel spectra at about the same time.
-template <int P>
+// Where parents have few children most of the 27 kernel spectra serve no pair: not
+// FULL reads a source's spectrum once, and a kernel spectrum for each target that
+// has it, which needs fewer registers too (5 waves per SIMD).  From kUnifFull
+// children per parent FULL is faster, M2L in us, few / full, uniform particles at
+// order 7: 1.1 children (5,000, h7) 1,141 / 2,468; 2.7 (100,000, h7) 14,804 / 23,991;
+// 4.2 (192,000, h7) 21,390 / 28,248; 5.5 (38,400, h6) 3,997 / 3,776; 8 (20,000, h5)
+// 815 / 582; a sphere of 30,000 at h8 2,418 / 5,260 (one target at a time 3,597).
+constexpr int64_t kUnifFull = 5;
+
+template <int P, bool FULL>
 __global__ __launch_bounds__(256) void k_unif_m2l(UnifLevels lv, const int16_t* __restrict__ slotpos,
                                                   const double2* __restrict__ K) {
     constexpr int N = 2 * P - 1, NF = P * N * N;
@@ -382,12 +391,14 @@ __global__ __launch_bounds__(256) void k_unif_m2l(UnifLevels lv, const int16_t* 
         const int c0 = cell0 + __builtin_amdgcn_readfirstlane(__builtin_ctzll(heads));
         const uint64_t parent = keys[c0] >> 3;
         int child[8];  // target cells by child index
+        uint32_t there = 0;
 #pragma unroll
         for (int a = 0; a < 8; ++a) child[a] = -1;
         for (int i = lane; i < 8 * kDirs; i += 64) src[i] = -1;
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");  // the wave's LDS accesses run in order
         for (int c = c0; c < nc && c < c0 + 8 && (keys[c] >> 3) == parent; ++c) {
             const int par = __builtin_amdgcn_readfirstlane(static_cast<int>(keys[c] & 7u));
+            there |= 1u << par;
 #pragma unroll
             for (int a = 0; a < 8; ++a)
                 if (a == par) child[a] = c;
@@ -408,14 +419,40 @@ __global__ __launch_bounds__(256) void k_unif_m2l(UnifLevels lv, const int16_t* 
         for (int a = 0; a < 8; ++a) acc[a] = make_double2(0., 0.);
         for (int dir = 0; dir < kDirs; ++dir) {
             const int at = lane < 8 ? src[8 * dir + lane] : -1;
-            if (__ballot(at >= 0) == 0) continue;  // no source there (nor in the parent itself)
+            uint32_t srcs = static_cast<uint32_t>(__ballot(at >= 0));
+            if (srcs == 0) continue;  // no source there (nor in the parent itself)
+            const int dx = dir / 9 - 1, dy = (dir / 3) % 3 - 1, dz = dir % 3 - 1;
+            if constexpr (!FULL) {
+#pragma unroll 1
+                for (; srcs; srcs &= srcs - 1) {
+                    const int b = __builtin_ctz(srcs);
+                    const double2 x = Mh[static_cast<int64_t>(__builtin_amdgcn_readlane(at, b)) * NF + fr];
+                    double2 k[8];
+                    uint32_t far = 0;  // targets that have b among their sources
+#pragma unroll
+                    for (int a = 0; a < 8; ++a) {
+                        if (!(there >> a & 1)) continue;
+                        const int px = 2 * dx + ((b >> 2) & 1) - ((a >> 2) & 1), py = 2 * dy + ((b >> 1) & 1) - ((a >> 1) & 1),
+                                  pz = 2 * dz + (b & 1) - (a & 1);
+                        if (abs(px) <= 1 && abs(py) <= 1 && abs(pz) <= 1) continue;  // near pairs
+                        far |= 1u << a;
+                        k[a] = K[static_cast<int64_t>(((px + 3) * 7 + py + 3) * 7 + pz + 3) * NF + fr];
+                    }
+#pragma unroll
+                    for (int a = 0; a < 8; ++a) {
+                        if (!(far >> a & 1)) continue;
+                        acc[a].x = fma(k[a].x, x.x, fma(-k[a].y, x.y, acc[a].x));
+                        acc[a].y = fma(k[a].x, x.y, fma(k[a].y, x.x, acc[a].y));
+                    }
+                }
+                continue;
+            }
             double2 m[8];
 #pragma unroll
             for (int b = 0; b < 8; ++b) {
                 const int v = __builtin_amdgcn_readlane(at, b);
                 m[b] = v >= 0 ? Mh[static_cast<int64_t>(v) * NF + fr] : make_double2(0., 0.);
             }
-            const int dx = dir / 9 - 1, dy = (dir / 3) % 3 - 1, dz = dir % 3 - 1;
 #pragma unroll
             for (int ox = -1; ox <= 1; ++ox)
 #pragma unroll
@@ -492,11 +529,12 @@ int run_unif_m2l(Context* c) {
     const int lo = c->work_upper > c->top() ? c->work_upper : c->top();
     const int hi = c->work_lower - 1 < L ? c->work_lower - 1 : L;
     const int k = c->glob.k;
-    UnifLevels lv{};
-    lv.first[0] = 0;
+    UnifLevels full{}, few{};  // by the children that the level's parents have
     for (int l = lo; l <= hi; ++l) {
         const int64_t nc = c->ncell[l];
         if (nc == 0) continue;
+        const int below = l == c->top() && l < L ? l + 1 : l;  // the top level goes with the one below it
+        UnifLevels& lv = c->ncell[below] >= kUnifFull * c->ncell[below - 1] ? full : few;
         const int i = lv.nlev++;
         lv.scale[i] = 2. / (c->P.box_width / static_cast<double>(int64_t(1) << (l - c->set_levels)));
         lv.slots[i] = c->d_m2l.as<int32_t>() + static_cast<size_t>(c->m2l_off[l]) * kFarSlots;
@@ -506,14 +544,19 @@ int run_unif_m2l(Context* c) {
         lv.ncell[i] = static_cast<int>(nc);
         lv.first[i + 1] = lv.first[i] + (nc + kUnifCells - 1) / kUnifCells;
     }
-    if (lv.nlev == 0) return HFMM_OK;
     const int16_t* sp = c->d_slotpos.as<int16_t>();
     const double2* K = reinterpret_cast<const double2*>(c->d_uK.as<double>());
     const int N = 2 * c->ops.p - 1, NF = c->ops.p * N * N;
-    const dim3 grid(static_cast<unsigned>(lv.first[lv.nlev]), static_cast<unsigned>((NF + 63) / 64));
+    const auto grid = [&](const UnifLevels& lv) {
+        return dim3(static_cast<unsigned>(lv.first[lv.nlev]), static_cast<unsigned>((NF + 63) / 64));
+    };
     prof_begin(c, "unif_m2l");
     switch (c->ops.p) {
-#define CASE(PP) case PP: hipLaunchKernelGGL(k_unif_m2l<PP>, grid, dim3(256), 0, c->stream, lv, sp, K); break;
+#define CASE(PP)                                                                                                          \
+    case PP:                                                                                                              \
+        if (full.nlev) hipLaunchKernelGGL((k_unif_m2l<PP, true>), grid(full), dim3(256), 0, c->stream, full, sp, K);      \
+        if (few.nlev) hipLaunchKernelGGL((k_unif_m2l<PP, false>), grid(few), dim3(256), 0, c->stream, few, sp, K);        \
+        break;
         HFMM_UNIF_ORDERS(CASE)
 #undef CASE
         default: prof_end(c); return fail(c, HFMM_ERR_ARG, "uniform M2L: unsupported order");
