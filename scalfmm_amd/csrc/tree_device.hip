@@ -845,6 +845,32 @@ __global__ __launch_bounds__(kBlock) void k_item_claims(int64_t cap, const int32
     for (int p = 0; p < k; ++p) claims[off[i] + p] = static_cast<int32_t>(i) * kP2PMaxParts + p;
 }
 
+// Both and the scan between them by one workgroup, for few items (claims has room
+// for every part): three launches were 50 of the 280 us of a build of 32 leaves.
+constexpr int64_t kClaimsOne = 2 * kTile;
+
+__global__ __launch_bounds__(kBlock) void k_claims_one(const int32_t* __restrict__ nitems, const int2* __restrict__ items,
+                                                      const int32_t* __restrict__ parts, int32_t* __restrict__ claims,
+                                                      int32_t* __restrict__ total) {
+    __shared__ int32_t sh[kBlock];
+    const int n = *nitems;
+    int32_t at = 0;
+    for (int i0 = 0; i0 < n; i0 += kTile) {
+        int32_t k[kItems], sum = 0;
+        const int i = i0 + static_cast<int>(threadIdx.x) * kItems;
+        for (int r = 0; r < kItems; ++r) {
+            k[r] = i + r < n ? parts[items[i + r].x] : 0;
+            sum += k[r];
+        }
+        int32_t tot;
+        int32_t to = at + block_exclusive_scan<int32_t>(sum, sh, tot);
+        for (int r = 0; r < kItems; ++r)
+            for (int p = 0; p < k[r]; ++p) claims[to++] = (i + r) * kP2PMaxParts + p;
+        at += tot;
+    }
+    if (threadIdx.x == 0) *total = at;
+}
+
 }  // namespace
 
 int m2l_slot_counts(Context* c, int level, unsigned long long* counts) {
@@ -1116,14 +1142,22 @@ int build_p2p_mutual_tables(Context* c, int64_t nbig) {
     HFMM_TRY(check_launch(c, "p2p_items"));
     HFMM_TRY(exclusive_scan<int64_t>(c, base, base, nl, p2p_mutual_units(c), "p2p_items"));
     const int64_t cap = c->p2p_items_m_cap;
+    const bool one = cap <= kClaimsOne;
     if (!is_mixed(c)) {
-        HFMM_TRY(ensure(c, c->d_scan, sizeof(int32_t) * static_cast<size_t>(cap)));
         prof_begin(c, "p2p_items");
-        hipLaunchKernelGGL(k_item_parts, dim3(blocks_for(cap)), dim3(kBlock), 0, c->stream, cap, p2p_mutual_item_count(c),
-                           c->d_p2pitems_m.as<int2>(), c->d_csparts.as<int32_t>(), c->d_scan.as<int32_t>());
+        if (one) {
+            HFMM_TRY(ensure(c, c->d_claims, sizeof(int32_t) * kP2PMaxParts * static_cast<size_t>(cap)));
+            hipLaunchKernelGGL(k_claims_one, dim3(1), dim3(kBlock), 0, c->stream, p2p_mutual_item_count(c),
+                               c->d_p2pitems_m.as<int2>(), c->d_csparts.as<int32_t>(), c->d_claims.as<int32_t>(), p2p_claim_count(c));
+        } else {
+            HFMM_TRY(ensure(c, c->d_scan, sizeof(int32_t) * static_cast<size_t>(cap)));
+            hipLaunchKernelGGL(k_item_parts, dim3(blocks_for(cap)), dim3(kBlock), 0, c->stream, cap, p2p_mutual_item_count(c),
+                               c->d_p2pitems_m.as<int2>(), c->d_csparts.as<int32_t>(), c->d_scan.as<int32_t>());
+        }
         prof_end(c);
         HFMM_TRY(check_launch(c, "p2p_items"));
-        HFMM_TRY(exclusive_scan<int32_t>(c, c->d_scan.as<int32_t>(), c->d_scan.as<int32_t>(), cap, p2p_claim_count(c), "p2p_items"));
+        if (!one)
+            HFMM_TRY(exclusive_scan<int32_t>(c, c->d_scan.as<int32_t>(), c->d_scan.as<int32_t>(), cap, p2p_claim_count(c), "p2p_items"));
     }
     int64_t counts[2] = {0, 0};  // units, claims
     HFMM_HIP(c, hipMemcpyAsync(counts, p2p_mutual_units(c), sizeof(counts), hipMemcpyDeviceToHost, c->stream));
@@ -1138,8 +1172,8 @@ int build_p2p_mutual_tables(Context* c, int64_t nbig) {
         if (bytes > (free_b + c->d_cpart.bytes) / 4) return HFMM_OK;  // ordered-pair kernel instead
     }
     HFMM_TRY(ensure(c, c->d_cpart, bytes));
-    if (!is_mixed(c)) {
-        c->p2p_claims = static_cast<int32_t>(counts[1]);
+    if (!is_mixed(c)) c->p2p_claims = static_cast<int32_t>(counts[1]);
+    if (!is_mixed(c) && !one) {
         HFMM_TRY(ensure(c, c->d_claims, sizeof(int32_t) * static_cast<size_t>(c->p2p_claims)));
         prof_begin(c, "p2p_items");
         hipLaunchKernelGGL(k_item_claims, dim3(blocks_for(cap)), dim3(kBlock), 0, c->stream, cap, p2p_mutual_item_count(c),
