@@ -7,7 +7,8 @@ from scalfmm_amd import _abi
 
 @contextlib.contextmanager
 def all_but(left):
-    """Holds the free device memory except about `left` bytes (at most: the largest piece that is left)."""
+    """Holds the free device memory except about `left` bytes; 0: all that the
+    runtime gives in pieces of 4 MiB, whatever it says is free (it keeps some of its own)."""
     hip = _abi.lib()  # the runtime that the engine is bound to
     free, total = ctypes.c_size_t(), ctypes.c_size_t()
     held = []
@@ -25,7 +26,7 @@ def all_but(left):
             while True:
                 if hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)):
                     raise RuntimeError("hipMemGetInfo")
-                if free.value < left + size or not take(size):
+                if (left and free.value < left + size) or not take(size):
                     break
         yield free.value
     finally:
