@@ -29,11 +29,13 @@
 // 21, 21, 21 per 16 rows).  A step is 32 (row, cell) lines of 16; the tile that
 // holds the Hadamard operands is double buffered, one barrier per step.
 //
-// Bound by the SIMDs: MFMAs 45-50% of the time, and FP64 MFMAs and VALU
-// instructions do not overlap (4 VALU instructions beside a 66-cycle MFMA add 16
-// cycles); the rest is the transform's VALU work and waits at the barriers.  1M
-// uniform particles, h7, order 7: 55.7 (one operator per slot) -> 15.8 ms, 33.9
-// TFLOP/s executed; 10M Plummer, h8, order 8: 202 -> 42 ms.
+// Of the SIMD cycles, MFMAs take 43% upward and 59% downward (1M uniform, h7, order
+// 7), VALU instructions 11% and 16% more: the two do not overlap (4 VALU
+// instructions beside a 66-cycle FP64 MFMA add 16 cycles).  The rest is waiting:
+// one workgroup of 8 waves fits a CU at orders 7 and 8 and has a barrier per step,
+// and upward every thread masks and stores 8 sums of 8 bytes per step.  1M uniform
+// particles, h7, order 7: 55.7 (one operator per slot) -> 15.8 ms, 33.9 TFLOP/s
+// executed; 10M Plummer, h8, order 8: 202 -> 42 ms.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
