@@ -1144,13 +1144,13 @@ int build_p2p_mutual_tables(Context* c, int64_t nbig) {
     const int64_t cap = c->p2p_items_m_cap;
     const bool one = cap <= kClaimsOne;
     if (!is_mixed(c)) {
+        if (one) HFMM_TRY(ensure(c, c->d_claims, sizeof(int32_t) * kP2PMaxParts * static_cast<size_t>(cap)));
+        else HFMM_TRY(ensure(c, c->d_scan, sizeof(int32_t) * static_cast<size_t>(cap)));
         prof_begin(c, "p2p_items");
         if (one) {
-            HFMM_TRY(ensure(c, c->d_claims, sizeof(int32_t) * kP2PMaxParts * static_cast<size_t>(cap)));
             hipLaunchKernelGGL(k_claims_one, dim3(1), dim3(kBlock), 0, c->stream, p2p_mutual_item_count(c),
                                c->d_p2pitems_m.as<int2>(), c->d_csparts.as<int32_t>(), c->d_claims.as<int32_t>(), p2p_claim_count(c));
         } else {
-            HFMM_TRY(ensure(c, c->d_scan, sizeof(int32_t) * static_cast<size_t>(cap)));
             hipLaunchKernelGGL(k_item_parts, dim3(blocks_for(cap)), dim3(kBlock), 0, c->stream, cap, p2p_mutual_item_count(c),
                                c->d_p2pitems_m.as<int2>(), c->d_csparts.as<int32_t>(), c->d_scan.as<int32_t>());
         }
