@@ -1109,6 +1109,20 @@ int ensure_parity_order(Context* c) {
     return HFMM_OK;
 }
 
+// Bytes that the first evaluation of the built tree takes beside what the context
+// has: expansions, results, and the M2L's least workspace (FP64 products: a step
+// of rows, 1 KB per cell, partial locals, up to 4, and what the pages round up; tiles:
+// multipoles in FP32).
+static size_t evaluation_needs(const Context* c) {
+    const auto lacks = [](const DevBuf& b, size_t bytes) { return bytes > b.bytes ? bytes - b.bytes : 0; };
+    const size_t exp = sizeof(double) * static_cast<size_t>(c->total_cells + 1) * c->LD;
+    const size_t values = sizeof(double) * static_cast<size_t>(c->n) * c->nrhs;
+    const size_t work = static_cast<size_t>(c->total_cells) * 6144;
+    const size_t own = c->d_m2lC.bytes + c->d_m2lacc.bytes;
+    return lacks(c->d_M, exp) + lacks(c->d_L, exp) + lacks(c->d_res_sorted, 4 * values) + lacks(c->d_res, 4 * values) +
+           lacks(c->d_field, 3 * values) + (work > own ? work - own : 0);
+}
+
 int build_p2p_mutual_tables(Context* c, int64_t nbig) {
     c->p2p_mutual = false;
     const int64_t nl = c->ncell[c->height() - 1];
@@ -1169,7 +1183,10 @@ int build_p2p_mutual_tables(Context* c, int64_t nbig) {
     if (bytes > c->d_cpart.bytes) {
         size_t free_b = 0, total_b = 0;
         HFMM_HIP(c, hipMemGetInfo(&free_b, &total_b));
-        if (bytes > (free_b + c->d_cpart.bytes) / 4) return HFMM_OK;  // ordered-pair kernel instead
+        free_b += c->d_cpart.bytes;
+        const size_t later = evaluation_needs(c);
+        // ordered-pair kernel instead
+        if (later > free_b || bytes > free_b / 4 || bytes > free_b - later) return HFMM_OK;
     }
     HFMM_TRY(ensure(c, c->d_cpart, bytes));
     if (!is_mixed(c)) c->p2p_claims = static_cast<int32_t>(counts[1]);

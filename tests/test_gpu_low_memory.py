@@ -77,3 +77,36 @@ def test_fp64_m2l_with_little_memory(n, h, order, cells, left):
     for a, b in zip(e.results(), ref):
         assert np.array_equal(a, b)
     e.close()
+
+
+def test_near_field_leaves_room_for_the_expansions():
+    """The slots of the near field (80 MB) would fit a quarter of the free
+    memory, but not beside the expansions (270 MB) and what the M2L needs at the
+    least (160 MB): the pairs are taken one way instead, within the FP64 path's 1e-12."""
+    from device_memory import all_but
+    from scalfmm_amd import Engine
+    from scalfmm_amd.distributions import uniform_cube
+    x, y, z, q = uniform_cube(90000, 7)
+    for a in (x, y, z):  # eight leaves of 3,750 particles
+        a[:30000] = 0.5 + (a[:30000] - 0.5) / 16
+
+    def engine(h):
+        e = Engine(h, 1.0, CENTER, 8)
+        e.set_particles(x, y, z, q)
+        return e
+
+    e = engine(6)
+    e.build_tree()
+    e.evaluate()
+    ref = e.results()
+    e.close()
+    e = engine(6)
+    e.synchronize()
+    with all_but(490 << 20) as left:
+        print("left", left, flush=True)
+        e.build_tree()
+        e.evaluate()
+        got = e.results()
+    for a, b in zip(got, ref):
+        assert np.linalg.norm(a - b) <= 1e-12 * np.linalg.norm(b)
+    e.close()
